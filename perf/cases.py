@@ -99,14 +99,14 @@ def draw(rng):
         return {"kind": "decode", "dtype": dtype, "batch": _spread(rng, 1, 256), "tokens": tokens, "heads": heads,
                 "key_dim": key_dim, "value_dim": value_dim, "in_place": tokens == 1 and rng.random() < 0.5}
     if kind == "cache":
-        return {"kind": "cache", "layers": rng.randint(1, 8), "batch": _spread(rng, 2, 64), "heads": heads,
+        return {"kind": "cache", "layers": rng.randint(1, 8), "batch": _spread(rng, 3, 64), "heads": heads,
                 "key_dim": key_dim, "value_dim": value_dim}
     if kind == "layer":
         use = rng.choice(["decode", "prefill", "train"])
-        batch = _spread(rng, 1, 128) if use == "decode" else rng.randint(1, 4)
+        batch = _spread(rng, 4, 256) if use == "decode" else rng.randint(1, 4)
         tokens = 1 if use == "decode" else _spread(rng, 65, 8192) // batch + 1
         return {"kind": "layer", "use": use, "dtype": "bf16", "batch": batch, "tokens": tokens,
-                "heads": rng.choice([8, 12, 16]), "key_dim": rng.choice([64, 128]), "value_dim": 128,
+                "heads": rng.choice([4, 6, 8, 10, 12, 14, 16]), "key_dim": rng.choice([64, 128]), "value_dim": 128,
                 "padded": use != "decode" and batch > 1 and rng.random() < 0.5}
     if kind == "train":
         count = rng.choice([1, 1, 2, 4])
