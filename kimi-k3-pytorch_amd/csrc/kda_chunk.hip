@@ -1943,44 +1943,83 @@ struct Plan {
 static std::atomic<int64_t> g_segment_override{-1};
 static int64_t segment_override() { return g_segment_override.load(std::memory_order_relaxed); }
 
+// The plan minimises a model of the call's time in microseconds, fitted to
+// graph-captured calls on one MI355X (B x H from 4 to 128, T from 100 to 4096,
+// K = V = 128, L forced from 0 to 16; K = V = 64 runs 0.85 times as long with
+// the same order):
+//   one segment per sequence: kUnsegChunk per chunk of the longest chain;
+//   L chunks per segment: the chunk steps of phases A and C together
+//   (kSegChunk) and a start-up (kSegStart) per round of workgroups, one
+//   combine step (kCombineStep) per segment of the longest chain, and the
+//   segment records' traffic (kSegBytes per segment and head: about 320 KB
+//   at V = 128 written and read back).
+// Both sides of the line, measured (us): B x H = 4, n = 6 chunks: unsegmented
+// 49.6, L = 1 28.6; n = 2: 20.8 against 23.7; n = 3: 28.1 against 27.3 (a cut
+// has to promise a tenth, kCutGain, or the chain stays whole); B x H = 16, n = 16: 123, L = 1
+// 44.6, L = 2 43.6; B x H = 4, n = 64: 466, L = 1 64.9, L = 2 56.1; B x H = 128,
+// n = 6: 52.7, L = 3 53.9.  (The rule before cut a sequence only past two
+// chunk-workgroups per CU, which left B x H = 4, T = 4096 at 466 us.)
+constexpr double kUnsegChunk = 7.3, kUnsegStart = 6.5, kCutGain = 0.9;
+constexpr double kSegChunk = 11.0, kSegStart = 6.0, kSegLaunches = 7.5, kCombineStep = 0.45, kSegBytes = 0.05;
+
 // `longest` (packed documents only, 0 when unknown): the longest document in
 // tokens.  Documents of uneven length that alone fill the GPU would leave it
-// idle while the longest runs on (one workgroup per document and head): when
-// the longest document is well past the chunk-steps per CU of a balanced
-// pass, every document is cut into segments of that many chunks (short ones
-// stay one segment), which spreads the long chains over the CUs the short
-// documents free.
+// idle while the longest runs on (one workgroup per document and head); cut
+// into segments, the long chains spread over the CUs the short documents free.
+// Past kModelledSteps chunk steps per CU the model's best is the balanced
+// pass, L = the chunk steps per CU, so no other length is priced there.
+constexpr int64_t kModelledSteps = 16;
 static Plan make_plan(int64_t N, int64_t total_tokens, int64_t H, int64_t V, int64_t longest) {
   Plan p;
   p.ncg = (V + kColGroup - 1) / kColGroup;
   const int64_t cus = device_cus();
   const int64_t chunks_bound = total_tokens / kChunk + N;
   p.chunks_bound = chunks_bound;
-  const int64_t work = (total_tokens / kChunk) * H * p.ncg;  // chunk-workgroups of one pass
+  auto segments_of = [&](int64_t L) {
+    p.L = static_cast<int32_t>(L < kOneSegment ? L : kOneSegment - 1);
+    p.segmented = true;
+    p.segs_bound = chunks_bound / p.L + N + 1;
+  };
   const int64_t forced = segment_override();
   if (forced > 0) {
-    p.L = static_cast<int32_t>(forced < kOneSegment ? forced : kOneSegment - 1);
-    p.segmented = true;
-    p.segs_bound = chunks_bound / p.L + N + 1;
+    segments_of(forced);
     return p;
   }
-  const int64_t per_cu = (work + cus - 1) / cus;  // chunk-steps per CU of a balanced pass
-  const int64_t longest_chunks = (longest + kChunk - 1) / kChunk;
-  const bool uneven = forced != 0 && N > 1 && per_cu >= 2 && 4 * longest_chunks > 5 * per_cu;
-  if (uneven && work >= 2 * cus) {
-    p.L = static_cast<int32_t>(per_cu < kOneSegment ? per_cu : kOneSegment - 1);
-    p.segmented = true;
-    p.segs_bound = chunks_bound / p.L + N + 1;
-  } else if (forced == 0 || N * H * p.ncg * 4 >= cus * 3 || work < 2 * cus) {
-    p.L = kOneSegment;
-    p.segmented = false;
-    p.segs_bound = N;
-  } else {
-    int64_t L = (work + cus - 1) / cus;
-    if (L < 2) L = 2;
-    p.L = static_cast<int32_t>(L);
-    p.segmented = true;
-    p.segs_bound = chunks_bound / L + N + 1;
+  p.L = kOneSegment;
+  p.segmented = false;
+  p.segs_bound = N;
+  if (forced == 0 || N <= 0) return p;
+  const int64_t span = longest > 0 ? longest : (total_tokens + N - 1) / N;  // the longest sequence (known or even)
+  const int64_t n = (span + kChunk - 1) / kChunk;                           // its chunks
+  const bool even = N * span <= total_tokens;
+  const double total = even ? static_cast<double>(N * n) : static_cast<double>(total_tokens / kChunk);
+  const double wgs = static_cast<double>(H * p.ncg);
+  const double steps = total * wgs / cus;  // chunk steps per CU of a balanced pass
+  // one chain per (sequence, head, column group) on three quarters of the CUs
+  // or more: cutting equal chains only adds a second round and the records
+  if (even && 4 * N * H * p.ncg >= 3 * cus) return p;
+  const double rounds0 = even ? static_cast<double>((N * H * p.ncg + cus - 1) / cus) * n : steps;
+  double best = kCutGain * (kUnsegStart + kUnsegChunk * (n > rounds0 ? n : rounds0));
+  const int64_t L1 = steps <= 1 ? 1 : static_cast<int64_t>(steps + 0.999);
+  const int64_t last = L1 <= kModelledSteps ? 4 * L1 + 4 : L1;
+  for (int64_t L = L1 <= kModelledSteps ? 1 : L1; L <= last && L < n; ++L) {
+    const int64_t nseg = (n + L - 1) / L;
+    double segs, waves, run;  // segments, rounds of workgroups, chunk steps per CU
+    if (even) {
+      segs = static_cast<double>(N * nseg);
+      waves = static_cast<double>((N * nseg * H * p.ncg + cus - 1) / cus);
+      run = waves * L;
+    } else {
+      segs = total / L + 0.5 * N;
+      waves = segs * wgs / cus > 1 ? segs * wgs / cus : 1;
+      run = L > steps ? L : steps;
+    }
+    const double us = kSegLaunches + kSegStart * waves + kSegChunk * run + kCombineStep * nseg +
+                      kSegBytes * segs * H * (static_cast<double>(V) / kColGroup);
+    if (us < best) {
+      best = us;
+      segments_of(L);
+    }
   }
   return p;
 }
