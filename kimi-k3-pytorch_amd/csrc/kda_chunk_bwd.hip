@@ -12,17 +12,18 @@
 // the backward is
 //   dVt = Kt dS' + Aqk^T dO,   dS = D dS' + Qg^T dO - W^T dVt,
 //   dQg = dO S^T, dAqk = tril(dO Vt^T), dKt = Vt dS'^T, dD = rowsum(dS' * S),
-//   dW = -dVt S^T, dv = M^T dVt, dM = dVt v^T + dW Kg^T, dKg = M^T dW,
-//   db_j = sum_i N_ij dM_ij + sum_k dL_jk A_jk,  dL = -strict(N^T dM diag(b) N^T),
-//   dA = diag(b) dL, then the pair sums of dA and dAqk with exact exponents,
-//   the exp factors, and dg = reverse cumulative sum of d lg over the chunk.
+//   E = N^T dVt, dv = diag(b) E, dKg = -dv S^T, dA = -strict(dv Vt^T),
+//   db_i = E_i . e_i (Vt = diag(b) e; see grad_kernel),
+//   then the pair sums of dA and dAqk with exact exponents, the exp factors,
+//   and dg = reverse cumulative sum of d lg over the chunk.
 //
-// f32 accumulation everywhere.  pair and prep's inverse and W, U products
-// multiply on the f32 MFMA (v_mfma_f32_16x16x4f32); prep's decay products A
-// and Aqk, the state scans and grad's slab products use split-bf16 operands on v_mfma_f32_16x16x32_bf16 (x = hi + lo, hi = bf16(x),
+// f32 accumulation everywhere.  The pair sums, E and prep's inverse multiply on
+// the f32 MFMA (v_mfma_f32_16x16x4f32); prep's decay products A and Aqk and its
+// W and U, the state scans and grad_kernel's slab products use split-bf16
+// operands on v_mfma_f32_16x16x32_bf16 (x = hi + lo, hi = bf16(x),
 // lo = bf16(x - hi); hi*hi + hi*lo + lo*hi, dropping terms of relative size
 // 2^-17), which keeps the f32-input gradients within about 1e-5 of the f64
-// oracle.  For bf16 and f16 inputs the scans and grad's slab products take
+// oracle.  For bf16 and f16 inputs the scans and the slab products take
 // single bf16 operands (kSplitOps): their gradients, rounded to the input
 // type, stay within about 5e-3 of the oracle.  Decay products use a 16-row block factorisation on the MFMA, with
 // an exact pairwise-exponent path for chunks whose decays leave its range
@@ -34,9 +35,8 @@
 //   seg_combine_kernel  Vt) and the backward scan (dS', dVt per chunk, dS0),
 //                       side by side, each cut into segments whose affine
 //                       maps are composed (section "segmented state scans");
-//   grad_pair_kernel    one block per chunk: grad_body (dv, dbeta, and the records
-//                       dQg, dKt, dKg, dA, dAqk), then pair_body (the pair sums
-//                       and the final dq, dk, dg) on the records just written.
+//   grad_kernel         one block per chunk, two per CU for bf16 and f16
+//                       inputs: every gradient from the scans' records.
 // Intermediates live in a caller-owned f32 workspace, one record per
 // (sequence, head, chunk), followed by the scans' segment records.
 #include <math.h>
@@ -58,7 +58,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Offsets (floats) of one (sequence, head, chunk) record of the workspace.
 struct Layout {
   int Kp, Vp;  // K padded to 64 or 128, V to a multiple of 32
-  int64_t N, A, Aqkt, Wr, Wt, Ktr, Ktt, Qgt, Kg, U, D, S, Vt, dS, dVt, dQg, dKt, dKg, dA, dAqk, dD, per;
+  int64_t N, A, Aqkt, Wr, Wt, Ktr, Ktt, Qgt, U, D, live, S, Vt, dS, dVt, per;
   int hs;  // S, dS and Vt of the backward stored as bf16 (single-operand inputs)
 };
 
@@ -69,8 +69,8 @@ struct Layout {
 // nothing of the forward touches them.  `split` false (bf16 and f16 inputs,
 // kSplitOps): the scans' operand records hold their hi plane alone and, in
 // the backward, S, dS and Vt are bf16 (the gradient kernel reads them as bf16
-// operands), which takes the backward's record from 593 to 425 KiB at
-// K = V = 128.
+// operands), which takes the backward's record from 433 to 265 KiB at
+// K = V = 128.  A is written only for chunks with a row of zero beta.
 __host__ __device__ inline Layout make_layout(int64_t K, int64_t V, bool backward = true, bool split = true) {
   Layout L;
   L.Kp = K <= 64 ? 64 : 128;
@@ -80,7 +80,7 @@ __host__ __device__ inline Layout make_layout(int64_t K, int64_t V, bool backwar
   int64_t o = 0;
   L.hs = 0;
   if (!backward) {
-    L.N = L.A = L.Wt = L.Ktr = L.Kg = L.dS = L.dVt = L.dQg = L.dKt = L.dKg = L.dA = L.dAqk = L.dD = 0;
+    L.N = L.A = L.Wt = L.Ktr = L.live = L.dS = L.dVt = 0;
     L.Aqkt = o; o += sc;
     L.Wr = o; o += sk;
     L.Ktt = o; o += sk;
@@ -102,21 +102,25 @@ __host__ __device__ inline Layout make_layout(int64_t K, int64_t V, bool backwar
   L.Ktr = o; o += sk;
   L.Ktt = o; o += sk;
   L.Qgt = o; o += sk;
-  L.Kg = o; o += ck;
   L.U = o; o += cv;
   L.D = o; o += L.Kp;
+  L.live = o; o += kC;
   L.S = o; o += hv;
   L.Vt = o; o += hc;
   L.dS = o; o += hv;
   L.dVt = o; o += cv;
-  L.dQg = o; o += ck;
-  L.dKt = o; o += ck;
-  L.dKg = o; o += ck;
-  L.dA = o; o += cc;
-  L.dAqk = o; o += cc;
-  L.dD = o; o += L.Kp;
   L.per = (o + 63) / 64 * 64;  // 256-byte records
   return L;
+}
+
+// Floats per chunk that the workspace query answers with: a documented formula
+// that callers size buffers by (593 and 425 KiB at K = V = 128), of which the
+// record above takes the first 433 and 265 KiB.
+inline int64_t workspace_record(int64_t K, int64_t V, bool split) {
+  const int64_t Kp = K <= 64 ? 64 : 128, Vp = (V + 31) / 32 * 32;
+  const int64_t cc = kC * kC, ck = kC * Kp, cv = kC * Vp, kv = Kp * Vp, s = split ? 1 : 2;
+  const int64_t n = 4 * cc + cc / s + 5 * ck / s + 4 * ck + 2 * cv + cv / s + 2 * kv / s + 2 * Kp;
+  return (n + 63) / 64 * 64;
 }
 
 template <class IT>
@@ -223,36 +227,6 @@ struct Pick<false, T, F> {
   typedef F type;
 };
 
-// A split matrix in LDS with its reduction index contiguous: element (r, k)
-// at p[r * rs + k] (hi) and p[plane + r * rs + k] (lo); a right operand is
-// held as its transpose (row = output column).
-struct SMat {
-  const __bf16* p;
-  int plane, rs;
-};
-
-// acc += A[r0:r0+16, 0:kd] B[0:kd, c0:c0+16]; lane (i, g) carries k = k0 + 8g ..
-// k0 + 8g + 7 of row r0 + i of A and of column c0 + i of B; kd % 32 == 0.
-// SPLIT false: hi*hi alone (the lo planes are not read).
-template <bool SPLIT = true>
-__device__ __forceinline__ f32x4 mma3(f32x4 acc, SMat A, int r0, SMat B, int c0, int kd) {
-  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  const __bf16* pa = A.p + (r0 + i) * A.rs + 8 * g;
-  const __bf16* pb = B.p + (c0 + i) * B.rs + 8 * g;
-  for (int k0 = 0; k0 < kd; k0 += 32) {
-    const bf16x8 ah = *reinterpret_cast<const bf16x8*>(pa + k0);
-    const bf16x8 bh = *reinterpret_cast<const bf16x8*>(pb + k0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, acc, 0, 0, 0);
-    if constexpr (SPLIT) {
-      const bf16x8 al = *reinterpret_cast<const bf16x8*>(pa + A.plane + k0);
-      const bf16x8 bl = *reinterpret_cast<const bf16x8*>(pb + B.plane + k0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc, 0, 0, 0);
-    }
-  }
-  return acc;
-}
-
 // Split record in the workspace: n bf16 hi values, then n lo values.  Eight
 // consecutive values from element idx (a multiple of 8) as two 16-byte stores
 // (SPLIT false: the hi store alone).
@@ -315,6 +289,14 @@ __device__ __forceinline__ f32x4 mma_sb(f32x4 acc, Mat A, int r0, Mat B, int c0,
 __device__ __forceinline__ int64_t tok(const int64_t b, const int64_t t, const int64_t T, const int64_t H,
                                        const int64_t h) {
   return (b * T + t) * H + h;
+}
+
+// Row offsets inside a chunk are 32-bit: 64 rows of H x 128 elements.
+constexpr int64_t kMaxHeads = (1LL << 32) / (kC * 128) - 1;
+
+// Rows of the chunk at t0 inside the sequence (1..64).
+__device__ __forceinline__ int row_limit(int64_t t0, int64_t T) {
+  return static_cast<int>(T - t0 < kC ? T - t0 : kC);
 }
 
 // Four consecutive elements of an input row: loaded raw, converted later, so
@@ -381,46 +363,34 @@ struct RowTile {
   static constexpr int G = NCOL / 4, PER = kC * G / NT;
   static_assert(PER * NT == kC * G, "the tile must split evenly over the threads");
   typename Raw4<IT>::type v[PER];
+  // the chunk's first row as a uniform base, the lane's row and column as a
+  // 32-bit offset
   __device__ __forceinline__ void fetch(const IT* src, int64_t b, int64_t t0, int64_t T, int64_t H, int64_t h,
                                         int64_t X, int col0, int tid) {
+    const IT* base = src + tok(b, t0, T, H, h) * X + col0;
+    const unsigned step = static_cast<unsigned>(H * X);
+    const int last = row_limit(t0, T) - 1;
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
       const int item = tid + NT * it, r = item / G, c4 = (item % G) * 4;
-      const int64_t t = t0 + r < T ? t0 + r : T - 1;
-      v[it] = *reinterpret_cast<const typename Raw4<IT>::type*>(src + tok(b, t, T, H, h) * X + col0 + c4);
+      const unsigned off = static_cast<unsigned>(r < last ? r : last) * step + static_cast<unsigned>(c4);
+      v[it] = *reinterpret_cast<const typename Raw4<IT>::type*>(base + off);
     }
   }
   template <int RS>
   __device__ __forceinline__ void store(float* dst, int64_t t0, int64_t Tv, int tid) const {
+    const int rows = static_cast<int>(Tv - t0 < kC ? Tv - t0 : kC);  // may be <= 0: an all-padding chunk
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
       const int item = tid + NT * it, r = item / G, c4 = (item % G) * 4;
-      *reinterpret_cast<f32x4*>(&dst[r * RS + c4]) = t0 + r < Tv ? widen<IT>(v[it]) : zero4();
+      *reinterpret_cast<f32x4*>(&dst[r * RS + c4]) = r < rows ? widen<IT>(v[it]) : zero4();
     }
   }
 };
 
-// k, q and g rows of a chunk into LDS with one round trip to memory
-template <class IT, int KP, int NT>
-__device__ __forceinline__ void load_kqg(float* kS, float* qS, float* lgS, const Args<IT>& a, int64_t b, int64_t t0,
-                                         int64_t h, int tid, int64_t Tv) {
-  if (rows_fast(a.K, 0, KP)) {
-    RowTile<IT, KP, NT> rk, rq, rg;
-    rk.fetch(a.k, b, t0, a.T, a.H, h, a.K, 0, tid);
-    rq.fetch(a.q, b, t0, a.T, a.H, h, a.K, 0, tid);
-    rg.fetch(a.g, b, t0, a.T, a.H, h, a.K, 0, tid);
-    rk.template store<kRS>(kS, t0, Tv, tid);
-    rq.template store<kRS>(qS, t0, Tv, tid);
-    rg.template store<kRS>(lgS, t0, Tv, tid);
-  } else {
-    load_rows<IT, KP, kRS, NT>(kS, a.k, b, t0, a.T, a.H, h, a.K, 0, tid, Tv);
-    load_rows<IT, KP, kRS, NT>(qS, a.q, b, t0, a.T, a.H, h, a.K, 0, tid, Tv);
-    load_rows<IT, KP, kRS, NT>(lgS, a.g, b, t0, a.T, a.H, h, a.K, 0, tid, Tv);
-  }
-}
-
-// load_ws split in two (fetch into registers, store into LDS rows of stride
-// RS), so that the loads can go out ahead of the point where the tile is needed.
+// NROW x NCOL f32 of a workspace matrix (row stride ld, from column col0) in
+// registers (fetch), then LDS rows of stride RS (store): the loads go out ahead
+// of the point where the tile is needed.
 template <int NROW, int NCOL, int NT>
 struct WsTile {
   static constexpr int G = NCOL / 4, PER = NROW * G / NT;
@@ -442,25 +412,6 @@ struct WsTile {
     }
   }
 };
-
-// NROW x NCOL f32 from a workspace matrix (row stride ld, from column col0)
-// into LDS rows of stride RS.
-template <int NROW, int NCOL, int RS, int NT>
-__device__ __forceinline__ void load_ws(float* dst, const float* src, int ld, int col0, int tid) {
-  constexpr int G = NCOL / 4, PER = NROW * G / NT;
-  static_assert(PER * NT == NROW * G, "the tile must split evenly over the threads");
-  f32x4 v[PER];
-#pragma unroll
-  for (int it = 0; it < PER; ++it) {
-    const int item = tid + NT * it, r = item / G, c4 = (item % G) * 4;
-    v[it] = *reinterpret_cast<const f32x4*>(src + r * ld + col0 + c4);
-  }
-#pragma unroll
-  for (int it = 0; it < PER; ++it) {
-    const int item = tid + NT * it, r = item / G, c4 = (item % G) * 4;
-    *reinterpret_cast<f32x4*>(&dst[r * RS + c4]) = v[it];
-  }
-}
 
 // Decay products e^(lg_i - lg_j) (j <= i) are formed on the MFMA as
 // (x_i e^(lg_i - r)) (y_j e^(r - lg_j)) with r = lg at the first row of i's
@@ -513,13 +464,6 @@ __device__ __forceinline__ bool decay_risk(const float* lgS, int tid) {
     risky |= lgS[16 * I * RS + c] - lgS[(16 * I + 15) * RS + c] > kMaxBlockDecay;
   }
   return risky;
-}
-
-// True when the chunk needs the exact path; lg in LDS rows of stride kRS,
-// the raw g's sign having been folded into `nonneg` by the caller.
-template <int KP, int NT>
-__device__ __forceinline__ bool needs_exact(const float* lgS, bool nonneg, int tid) {
-  return __syncthreads_or(nonneg || decay_risk<KP, NT>(lgS, tid));
 }
 
 // accK += sum_c (k_i e^(lg_i - r)) (k_j e^(r - lg_j)) and accQ the same with
@@ -599,7 +543,7 @@ __device__ __forceinline__ int opaque(int x) {
 //   over the whole chunk);
 //   Kt = e^(lg_last - lg) k and Qg = e^lg q in place of q and lg, and
 //   Kg = e^lg k into a [64][KP] tile that stays for W = M Kg, with their
-//   records (D, Kg and Kt row-major, Kt^T, Qg^T).
+//   records (D, Kt row-major, Kt^T, Qg^T).
 // A chunk whose decays fall outside the factorisation's bounds repeats the
 // quarters for A and Aqk with exact pair exponents.  Then N = L^-1,
 // M = N diag(b), W = M Kg and U = M v.
@@ -631,6 +575,12 @@ struct QuarterTiles {
     }
   }
 };
+
+// A row whose beta is zero to f32 (its Vt = beta e underflows against e) still
+// has a beta gradient, E . e.  The backward's records hold e = v - Kg S - A Vt
+// itself on such rows (rows of U and W scaled by one instead of beta) and live
+// = 0, which keeps the row out of every product.
+__device__ __forceinline__ bool zero_beta(float b) { return !(fabsf(b) >= 0x1p-100f); }
 
 template <class IT, int KP>
 __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
@@ -667,15 +617,17 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     const int64_t n = a.valid[b];
     Tv = n < 0 ? 0 : (n < a.T ? n : a.T);
   }
-  // the records only the gradient kernels read (A, N, Kg, Kt row-major, W^T)
-  // are skipped when the kernels serve the forward alone (no dO)
+  // the records only the backward reads (N, Kt row-major, W^T, live) are
+  // skipped when the kernels serve the forward alone (no dO)
   const bool bwd_records = a.dout != nullptr;
 
   QuarterTiles<IT> in;
   in.fetch(a, b, t0, h, 0, tid);
   if (tid < kC) {
     const int64_t t = t0 + tid;
-    bS[tid] = t < Tv ? to_float(a.beta[tok(b, t, a.T, a.H, h)]) : 0.f;
+    const float x = t < Tv ? to_float(a.beta[tok(b, t, a.T, a.H, h)]) : 0.f;
+    bS[tid] = x;
+    if (bwd_records) ws[a.L.live + tid] = zero_beta(x) ? 0.f : 1.f;
   }
   for (int idx = tid; idx < kC * kRC; idx += kPT) AS[idx] = 0.f;
   // wave w: block pair w, and waves 0 and 1 pairs 8 and 9 as well
@@ -702,7 +654,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     }
     __syncthreads();
     // each element's factors once: Kt and Qg in place of q and lg, Kg into
-    // its tile, and the row-major Kg and Kt records written on the way
+    // its tile, and the row-major Kt record written on the way
     for (int i8 = tq; i8 < kC * kQC / 8; i8 += kPT) {
       const int r = (8 * i8) / kQC, cl = (8 * i8) % kQC;
       const float* kp = &kS[r * kQS + cl];
@@ -722,14 +674,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
           qg[4 * u + e] = ex * qq[e];
         }
       }
-      if (bwd_records) {  // Kg (f32) and Kt split, row-major
-        const int idx = r * KP + c0 + cl;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          *reinterpret_cast<f32x4*>(ws + a.L.Kg + idx + 4 * u) =
-              f32x4{kg[4 * u], kg[4 * u + 1], kg[4 * u + 2], kg[4 * u + 3]};
-        put_split8<kSplitOps<IT>>(ws + a.L.Ktr, kC * KP, idx, kt);
-      }
+      if (bwd_records) put_split8<kSplitOps<IT>>(ws + a.L.Ktr, kC * KP, r * KP + c0 + cl, kt);  // Kt row-major
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         *reinterpret_cast<f32x4*>(&KgS[r * kRS + c0 + cl + 4 * u]) =
@@ -753,6 +698,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     __syncthreads();
   }
   const bool exact = __syncthreads_or(risky);
+  const bool some_zero = bwd_records && __syncthreads_or(tid < kC && zero_beta(bS[tid & (kC - 1)]));
   if (exact) {
     // A and Aqk with exact pair exponents, 2x2 blocks of (i, j <= i): thread
     // tid takes blocks tid and tid + kPT of the 528, over the quarters again
@@ -854,7 +800,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
   __syncthreads();
   // per-lane addresses of the record stores formed here, not at the top
   const int tr = opaque(tid);
-  for (int i4 = tr; bwd_records && i4 < kC * kC / 4; i4 += kPT) {  // A, four at a time
+  for (int i4 = tr; some_zero && i4 < kC * kC / 4; i4 += kPT) {  // A, four at a time
     const int r = (4 * i4) >> 6, cc = (4 * i4) & 63;
     *reinterpret_cast<f32x4*>(ws + a.L.A + 4 * i4) = *reinterpret_cast<const f32x4*>(&AS[r * kRC + cc]);
   }
@@ -922,6 +868,27 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     *reinterpret_cast<f32x4*>(&AS[r * kRC + cc]) = n * *reinterpret_cast<const f32x4*>(&bS[cc]);
   }
   __syncthreads();
+  if (some_zero) {  // rows of zero beta: I - A M in place of M (thread: row tid / 8, columns 8 (tid % 8) ..)
+    const int i = tr >> 3, c8 = (tr & 7) * 8;
+    const bool zero = zero_beta(bS[i]);
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = c8 + e == i ? 1.f : 0.f;
+    if (zero) {
+#pragma unroll 1
+      for (int l = 0; l < i; ++l) {
+        const float al = ws[a.L.A + i * kC + l];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] -= al * AS[l * kRC + c8 + e];
+      }
+    }
+    __syncthreads();
+    if (zero) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) AS[i * kRC + c8 + e] = x[e];
+    }
+    __syncthreads();
+  }
   // W = M Kg, staged in f32 over Kg once every tile is formed
   f32x4 wt[NW];
 #pragma unroll
@@ -947,7 +914,13 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
       y[e] = KgS[(r2 + e) * kRS + c2];
     }
     put_split8<kSplitOps<IT>>(ws + a.L.Wr, kC * KP, 8 * i8, x);
-    if (bwd_records) put_split8<kSplitOps<IT>>(ws + a.L.Wt, kC * KP, 8 * i8, y);
+    if (bwd_records) {
+      if (some_zero) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = zero_beta(bS[r2 + e]) ? 0.f : y[e];
+      }
+      put_split8<kSplitOps<IT>>(ws + a.L.Wt, kC * KP, 8 * i8, y);
+    }
   }
   __syncthreads();
   if (v_early) {
@@ -1008,7 +981,8 @@ struct SegLds {
   static constexpr int fq = fb + ncol * 2048;   // backward Qg^T                 [KP][64]
   static constexpr int faq = fq + ncol * 2048;  // backward Aqk^T                [64][64]
   static constexpr int d = faq + 8 * 2048;      // D f32 [KP]
-  static constexpr int bytes = d + KP * 4;
+  static constexpr int live = d + KP * 4;      // live f32 [64] (the forward scan of a backward)
+  static constexpr int bytes = live + kC * 4;
 };
 
 // A split record [R][NC] of the workspace (R x NC bf16 hi, then lo; the hi
@@ -1179,7 +1153,7 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
   Rec<KP, kC, SPLIT> rb;   // forward Kt^T, backward W^T    [KP][64]
   Rec<KP, kC, SPLIT> rq;   // backward Qg^T
   Rec<kC, kC, SPLIT> raq;  // backward Aqk^T
-  float dval = 0.f;
+  float dval = 0.f, lval = 1.f;
   float u[4][4];    // forward value columns: U of the next chunk, accumulator layout
   DoFrag<IT> dof;   // backward value columns: dO of the next chunk
   auto chunk_of = [&](int p) -> int64_t { return BWD ? hi - 1 - p : lo + p; };
@@ -1194,6 +1168,7 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
       if (part == 1) {
         rb.fetch(ws + a.L.Ktt, tid);
         if (tid < KP) dval = ws[a.L.D + tid];
+        if (a.ndir == 2 && tid < kC) lval = ws[a.L.live + tid];
       }
       if (part == 2 && !TRANS && has) {
         const float* up = ws + a.L.U + opaque(4 * g4 * Vp + col);
@@ -1234,6 +1209,7 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
       raq.store(sm, SL::faq, tid);
     }
     if (tid < KP) reinterpret_cast<float*>(sm + SL::d)[tid] = dval;
+    if (!BWD && tid < kC) reinterpret_cast<float*>(sm + SL::live)[tid] = lval;
     float uc[4][4];
     bf16x8 doh[2], dol[2];
     if (!TRANS && has) {
@@ -1337,6 +1313,11 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
     // X' = D X + A^T R (forward A = Kt, backward A = W), plus Qg^T dO
     // (backward value columns); one fragment pair ahead
     bf16x8 rh[2], rl[2];
+    if constexpr (!BWD) {  // rows of zero beta hold e and write nothing
+#pragma unroll
+      for (int I = 0; I < 4; ++I)
+        P[I] *= *reinterpret_cast<const f32x4*>(sm + SL::live + (16 * I + 4 * g4) * 4);
+    }
 #pragma unroll
     for (int st = 0; st < 2; ++st) split_pair<SPLIT>(P[2 * st], P[2 * st + 1], rh[st], rl[st]);
     if (more) fetch_part(p + 1, 2);
@@ -1637,30 +1618,59 @@ __global__ __launch_bounds__(kOT) void out_kernel(const Args<IT> a) {
   }
 }
 
-// ---- grad_body: products that reduce over the state columns --------------------
-// Eight waves; slabs of 32 state columns accumulate dQg, dKt, dW (wave w:
-// row tile w % 4, half w / 4 of the column tiles),
-// dAqk and dM in MFMA accumulators and write dv; then dKg = M^T dW,
-// dM += dW Kg^T, dbeta and dA follow from N.
-constexpr int kSR = kSW + 8;                    // bf16 row stride of the split slab tiles
-constexpr int kOffM = 0;                        // [64][68] f32 M = N diag(b)
-constexpr int kOffSs = kOffM + kC * kRC;        // S slab split [128][kSR] x 2 planes (bf16; offsets in floats)
-constexpr int kOffdSn = kOffSs + 128 * kSR;     // dS' slab split
-constexpr int kOffdOs = kOffdSn + 128 * kSR;    // dO slab split [64][kSR] x 2
-constexpr int kOffVts = kOffdOs + kC * kSR;     // Vt slab split
-constexpr int kOffdVts = kOffVts + kC * kSR;    // dVt slab split
-constexpr int kOffvs = kOffdVts + kC * kSR;     // v slab split
-constexpr int kOffdVf = kOffvs + kC * kSR;      // dVt slab f32 [64][36] (the B operand of dv = M^T dVt)
-constexpr int kGradFloats = kOffdVf + kC * kSS;
-// second stage, over the slabs
-constexpr int kOffX = kOffSs;                   // [64][132] dW
-constexpr int kOffY = kOffX + kC * kRS;         // [64][132] Kg
-constexpr int kOffN = kOffSs;                   // [64][68]
-constexpr int kOffDM = kOffN + kC * kRC;        // [64][68] dM, then T1 = N^T dN
-constexpr int kOffDN = kOffDM + kC * kRC;       // [64][68] dN, then dL
-constexpr int kOffA = kOffDN + kC * kRC;        // [64][68]
-static_assert(kOffY + kC * kRS <= kGradFloats, "dW and Kg must fit");
-static_assert(kOffA + kC * kRC <= kGradFloats, "second-stage tiles must fit");
+// ---- grad_kernel: every gradient of a chunk from its scan records --------------
+// One workgroup per (sequence, head, chunk).  With E = N^T dVt (N = (I + diag(b)
+// A)^-1), the gradient through the chunk's triangular solve needs no product
+// with A, M or W:
+//   dv = diag(b) E,  dA = -strict(dv Vt^T),  dKg = -dv S^T,
+//   db_i = E_i . e_i  with Vt = diag(b) e  (e = v - Kg S - A Vt, the delta
+//   rule's error; a row whose b is zero to f32 holds e itself, see prep_kernel),
+// since dM = dVt (v - Kg S)^T makes dL = -strict(N^T dM diag(b) N^T)
+// = -strict(E Vt^T).  Beside these dQg = dO S^T, dAqk = tril(dO Vt^T),
+// dKt = Vt dS'^T, dD = rowsum(dS' * S).
+//
+// First stage, over slabs of 32 state columns: the products above, dQg, dKt and
+// dKg accumulated in MFMA registers (wave w: rows 16 (w / 2).., column tiles
+// 2 j + w % 2).  Second stage, over quarters of 32 key channels: the pair sums
+//   R1_i = sum_j dA_ij k_j E_ij,  R2_i = sum_j dAqk_ij k_j E_ij   (j <= i)
+//   R3_j = sum_i dA_ij k_i E_ij + sum_i dAqk_ij q_i E_ij           (i >= j)
+// on the f32 MFMA with the 16-row block factorisation of the decay (r_I = lg at
+// the first row of block I; a quarter outside its range takes exact pair
+// exponents), in the accumulator layout of the first stage, so that
+//   dq = e^(lg - r) R2 + e^lg dQg,  dk = [e^(lg - r) R1 + e^lg dKg] + [R3 + e^(lg_last - lg) dKt],
+//   d lg = k ([..] - [..]) + q dq  (+ sum(Kt dKt) + D dD on the last row)
+// and dg, its reverse cumulative sum, follow in registers.
+//
+// Bound: the latency of its phases (about 51 us a workgroup, 20 of it in the
+// slabs, 26 in the quarters); the 256 KB a chunk it must move at K = V = 128 for
+// bf16 would take 95 us over B = 1, T = 8192, H = 16.  66 KB of LDS and at most
+// 128 VGPRs let two workgroups share a CU for bf16 and f16 inputs (f32 inputs
+// keep hi and lo planes: one workgroup; so does bf16 at 256 VGPRs, 65 us slower
+// a call).  Measured there, bf16: 212 us against 354 for the two stages it
+// replaces (dM, dW and their products with N and A, one workgroup per CU, its
+// 144 KB of gradient records through memory); the whole backward 705 -> 549 us.
+constexpr int kGT = 512;                // threads of grad_kernel
+constexpr int kSR = kSW + 8;            // bf16 row stride of the slab tiles
+template <class IT, int KP>
+struct GradLds {
+  static constexpr int planes = kSplitOps<IT> ? 2 : 1;
+  static constexpr int NS = 0;                                // f32 [64][kRC]
+  static constexpr int S = NS + kC * kRC * 4;                 // bf16 planes x [KP][kSR]
+  static constexpr int dS = S + planes * KP * kSR * 2;        // the same
+  static constexpr int dO = dS + planes * KP * kSR * 2;       // bf16 planes x [64][kSR]
+  static constexpr int Vt = dO + planes * kC * kSR * 2;
+  static constexpr int dv = Vt + planes * kC * kSR * 2;
+  static constexpr int dVf = dv + planes * kC * kSR * 2;      // f32 [64][kSS]
+  static constexpr int slab_end = dVf + kC * kSS * 4;
+  // second stage, over the first
+  static constexpr int dA = 0;                                // f32 [64][kRC]
+  static constexpr int dAqk = dA + kC * kRC * 4;
+  static constexpr int k = dAqk + kC * kRC * 4;               // f32 [64][kQS]
+  static constexpr int q = k + kC * kQS * 4;
+  static constexpr int lg = q + kC * kQS * 4;
+  static constexpr int pair_end = lg + kC * kQS * 4;
+  static constexpr int bytes = slab_end > pair_end ? slab_end : pair_end;
+};
 
 // One slab tile (rows x 32 columns, f32 values v for columns c4..c4+3 of row r)
 // into a split tile of row stride kSR (bf16) and plane `plane` (SPLIT false:
@@ -1679,48 +1689,11 @@ __device__ __forceinline__ void put_split4(__bf16* dst, int plane, int r, int c4
   if constexpr (SPLIT) *reinterpret_cast<bf16x4*>(dst + plane + r * kSR + c4) = lo;
 }
 
-// A NROW x 32 workspace slab (row stride ld, from column col0), split into LDS.
-template <int NROW, int NT, bool SPLIT>
-__device__ __forceinline__ void load_ws_split(__bf16* dst, const float* src, int ld, int col0, int tid) {
-  constexpr int PER = NROW * 8 / NT;
-  static_assert(PER * NT == NROW * 8, "the tile must split evenly over the threads");
-  f32x4 v[PER];
-#pragma unroll
-  for (int it = 0; it < PER; ++it) {
-    const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-    v[it] = *reinterpret_cast<const f32x4*>(src + r * ld + col0 + c4);
-  }
-#pragma unroll
-  for (int it = 0; it < PER; ++it) {
-    const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-    put_split4<SPLIT>(dst, NROW * kSR, r, c4, v[it]);
-  }
-}
-
-// A NROW x 32 bf16 workspace slab (row stride ld, from column col0) into the
-// hi plane of a split tile.
-template <int NROW, int NT>
-__device__ __forceinline__ void load_ws_half(__bf16* dst, const float* src, int ld, int col0, int tid) {
-  constexpr int PER = NROW * 8 / NT;
-  static_assert(PER * NT == NROW * 8, "the tile must split evenly over the threads");
-  const __bf16* p = reinterpret_cast<const __bf16*>(src);
-  bf16x4 v[PER];
-#pragma unroll
-  for (int it = 0; it < PER; ++it) {
-    const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-    v[it] = *reinterpret_cast<const bf16x4*>(p + r * ld + col0 + c4);
-  }
-#pragma unroll
-  for (int it = 0; it < PER; ++it) {
-    const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-    *reinterpret_cast<bf16x4*>(dst + r * kSR + c4) = v[it];
-  }
-}
-
-// One 32-column slab of grad_body's operands in registers: the S and dS
-// rows (KP x 32), Vt and dVt (64 x 32, f32 from the workspace) and dO and v
-// (64 x 32 from the inputs; the whole-group case of load_rows_split).  The
-// next slab's loads go out while the current one is multiplied.
+// One 32-column slab of grad_kernel's operands in registers: the S and dS rows
+// (KP x 32), Vt and dVt (64 x 32, from the workspace, whose columns are padded)
+// and dO (64 x 32 from the input, element by element where its columns are not
+// whole 4-element groups inside V).  The next slab's loads go out while the
+// current one is multiplied.
 template <class IT, int KP, int NT>
 struct GradSlab {
   static constexpr int PS = KP * 8 / NT, PC = kC * 8 / NT;
@@ -1731,650 +1704,448 @@ struct GradSlab {
   typedef typename Pick<W32, f32x4, bf16x4>::type st_t;
   st_t s[PS], ds[PS], vt[PC];
   f32x4 dvt[PC];
-  typename Raw4<IT>::type dout[PC], v[PC];
-  __device__ __forceinline__ static st_t ld(const float* base, int idx) {
-    if constexpr (W32) return *reinterpret_cast<const f32x4*>(base + idx);
-    else return *reinterpret_cast<const bf16x4*>(reinterpret_cast<const __bf16*>(base) + idx);
+  typename Raw4<IT>::type dout[PC];
+  __device__ __forceinline__ static st_t ld(const float* base, int s0, unsigned off) {
+    if constexpr (W32) return *reinterpret_cast<const f32x4*>(base + s0 + off);
+    else return *reinterpret_cast<const bf16x4*>(reinterpret_cast<const __bf16*>(base) + s0 + off);
   }
   __device__ __forceinline__ static void put(__bf16* dst, int plane, int r, int c4, const st_t& x) {
     if constexpr (W32) put_split4<true>(dst, plane, r, c4, x);
     else *reinterpret_cast<bf16x4*>(dst + r * kSR + c4) = x;
   }
-  __device__ __forceinline__ void fetch(const Args<IT>& a, const float* ws, int64_t b, int64_t t0, int64_t h, int s0,
-                                        int tid) {
+  // dO0: the chunk's first row of dO, `step` elements to the next, `rows` of them real
+  __device__ __forceinline__ void fetch(const Args<IT>& a, const float* ws, const IT* dO0, unsigned step, int rows,
+                                        int s0, int tid, bool whole) {
     const int Vp = a.L.Vp;
 #pragma unroll
     for (int it = 0; it < PS; ++it) {
-      const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-      s[it] = ld(ws + a.L.S, r * Vp + s0 + c4);
-      ds[it] = ld(ws + a.L.dS, r * Vp + s0 + c4);
+      const int item = tid + NT * it;
+      const unsigned off = static_cast<unsigned>((item >> 3) * Vp + (item & 7) * 4);
+      s[it] = ld(ws + a.L.S, s0, off);
+      ds[it] = ld(ws + a.L.dS, s0, off);
     }
 #pragma unroll
     for (int it = 0; it < PC; ++it) {
       const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-      vt[it] = ld(ws + a.L.Vt, r * Vp + s0 + c4);
-      dvt[it] = *reinterpret_cast<const f32x4*>(ws + a.L.dVt + r * Vp + s0 + c4);
-      const int64_t t = t0 + r < a.T ? t0 + r : a.T - 1;
-      const int64_t row = tok(b, t, a.T, a.H, h) * a.V + s0 + c4;
-      dout[it] = *reinterpret_cast<const typename Raw4<IT>::type*>(a.dout + row);
-      v[it] = *reinterpret_cast<const typename Raw4<IT>::type*>(a.v + row);
+      const unsigned off = static_cast<unsigned>(r * Vp + c4);
+      vt[it] = ld(ws + a.L.Vt, s0, off);
+      dvt[it] = *reinterpret_cast<const f32x4*>(ws + a.L.dVt + s0 + off);
+      const unsigned row = static_cast<unsigned>(r < rows ? r : rows - 1) * step;
+      if (whole) {
+        dout[it] = *reinterpret_cast<const typename Raw4<IT>::type*>(dO0 + s0 + (row + static_cast<unsigned>(c4)));
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int col = s0 + c4 + u, V = static_cast<int>(a.V);
+          const IT x = dO0[row + static_cast<unsigned>(col < V ? col : V - 1)];
+          dout[it][u] = col < V ? x : static_cast<IT>(0.f);
+        }
+      }
     }
   }
-  __device__ __forceinline__ void store(__bf16* Ss, __bf16* dSn, __bf16* Vts, __bf16* dVts, float* dVf, __bf16* dOs,
-                                        __bf16* vs, int64_t t0, int64_t T, int tid) const {
+  // into LDS; dd[it] += this slab's part of row r's sum(dS' * S)
+  __device__ __forceinline__ void store(__bf16* Ss, __bf16* dSn, __bf16* Vts, float* dVf, __bf16* dOs, float (&dd)[PS],
+                                        int rows, int tid) const {
 #pragma unroll
     for (int it = 0; it < PS; ++it) {
       const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
       put(Ss, KP * kSR, r, c4, s[it]);
       put(dSn, KP * kSR, r, c4, ds[it]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dd[it] += static_cast<float>(s[it][e]) * static_cast<float>(ds[it][e]);
     }
 #pragma unroll
     for (int it = 0; it < PC; ++it) {
       const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
       put(Vts, kC * kSR, r, c4, vt[it]);
-      put_split4<W32>(dVts, kC * kSR, r, c4, dvt[it]);
       *reinterpret_cast<f32x4*>(&dVf[r * kSS + c4]) = dvt[it];
-      const bool real = t0 + r < T;
-      put_split4<W32>(dOs, kC * kSR, r, c4, real ? widen<IT>(dout[it]) : zero4());
-      put_split4<W32>(vs, kC * kSR, r, c4, real ? widen<IT>(v[it]) : zero4());
+      if constexpr (__is_same(IT, bf16)) {  // its own operand
+        typename Raw4<IT>::type x = dout[it];
+        if (r >= rows) x = typename Raw4<IT>::type{};
+        *reinterpret_cast<typename Raw4<IT>::type*>(dOs + r * kSR + c4) = x;
+      } else {
+        put_split4<W32>(dOs, kC * kSR, r, c4, r < rows ? widen<IT>(dout[it]) : zero4());
+      }
     }
   }
 };
 
-// Columns col0 .. col0+31 of the chunk's rows of an input [B,T,H,X], split into
-// LDS (zero past T and X); see load_rows.
-template <class IT, int NT>
-__device__ __forceinline__ void load_rows_split(__bf16* dst, const IT* src, int64_t b, int64_t t0, int64_t T,
-                                                int64_t H, int64_t h, int64_t X, int col0, int tid) {
-  constexpr int PER = kC * 8 / NT;
-  typedef typename Raw4<IT>::type raw_t;
-  if ((X & 3) == 0 && col0 + 32 <= X) {
-    raw_t v[PER];
-#pragma unroll
-    for (int it = 0; it < PER; ++it) {
-      const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-      const int64_t t = t0 + r < T ? t0 + r : T - 1;
-      v[it] = *reinterpret_cast<const raw_t*>(src + tok(b, t, T, H, h) * X + col0 + c4);
+// One 16-row fragment of a slab tile (row r0 + lane % 16, columns 8 (lane / 16) ..)
+template <bool SPLIT>
+struct SlabFrag {
+  bf16x8 hi, lo;
+  __device__ __forceinline__ void load(const __bf16* p, int plane, int r0, int li, int g4) {
+    const __bf16* x = p + (r0 + li) * kSR + 8 * g4;
+    hi = *reinterpret_cast<const bf16x8*>(x);
+    if constexpr (SPLIT) lo = *reinterpret_cast<const bf16x8*>(x + plane);
+  }
+  __device__ __forceinline__ void keep(bool live) {  // zeros when not live
+    if (!live) {
+      hi = bf16x8{};
+      if constexpr (SPLIT) lo = bf16x8{};
     }
+  }
+};
+template <bool SPLIT>
+__device__ __forceinline__ f32x4 mma_frag(const SlabFrag<SPLIT>& x, const SlabFrag<SPLIT>& y, f32x4 acc) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.hi, y.hi, acc, 0, 0, 0);
+  if constexpr (SPLIT) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.hi, y.lo, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.lo, y.hi, acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+// Four consecutive elements of one output row (columns col .. col + 3 of X) at dst + off.
+template <class IT>
+__device__ __forceinline__ void put_row4(IT* dst, unsigned off, int col, int X, bool whole, const f32x4& x) {
+  if (whole) {
+    typename Raw4<IT>::type y;
 #pragma unroll
-    for (int it = 0; it < PER; ++it) {
-      const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-      put_split4<kSplitOps<IT>>(dst, kC * kSR, r, c4, t0 + r < T ? widen<IT>(v[it]) : zero4());
-    }
+    for (int u = 0; u < 4; ++u) y[u] = from_compute<IT>(x[u]);
+    *reinterpret_cast<typename Raw4<IT>::type*>(dst + off) = y;
   } else {
-    for (int it = 0; it < PER; ++it) {
-      const int item = tid + NT * it, r = item >> 3, c4 = (item & 7) * 4;
-      const int64_t t = t0 + r;
-      f32x4 x = zero4();
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t col = col0 + c4 + u;
-        x[u] = (t < T && col < X) ? to_float(src[tok(b, t, T, H, h) * X + col]) : 0.f;
-      }
-      put_split4<kSplitOps<IT>>(dst, kC * kSR, r, c4, x);
+    for (int u = 0; u < 4; ++u)
+      if (col + u < X) dst[off + u] = from_compute<IT>(x[u]);
+  }
+}
+
+// The pair sums of one 16 x 16 tile (rows 16 J.., channel column cc of the
+// quarter) on the f32 MFMA; see grad_kernel.  R1, R2 come without their factor
+// e^(lg - r_J).
+__device__ __forceinline__ void pair_mfma(f32x4& R1, f32x4& R2, f32x4& R3, const float* kS, const float* qS,
+                                          const float* lgS, const float* dAS, const float* dQS, int J, int cc, int li,
+                                          int g4) {
+  const float rJ = lgS[16 * J * kQS + cc];
+  for (int b0 = 0; b0 <= J; ++b0) {  // rows j of block b0 <= J
+    float ak[4], aq[4], kj[4], lj[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = 16 * b0 + 4 * u + g4;
+      ak[u] = dAS[(16 * J + li) * kRC + j];
+      aq[u] = dQS[(16 * J + li) * kRC + j];
+      kj[u] = kS[j * kQS + cc];
+      lj[u] = lgS[j * kQS + cc];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float bk = kj[u] * fast_exp(rJ - lj[u]);
+      R1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ak[u], bk, R1, 0, 0, 0);
+      R2 = __builtin_amdgcn_mfma_f32_16x16x4f32(aq[u], bk, R2, 0, 0, 0);
+    }
+  }
+  for (int I = J; I < 4; ++I) {  // rows i of block I >= J
+    const float rI = lgS[16 * I * kQS + cc];
+    float ak[4], aq[4], ki[4], qi[4], l[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = 16 * I + 4 * u + g4;
+      ak[u] = dAS[i * kRC + 16 * J + li];
+      aq[u] = dQS[i * kRC + 16 * J + li];
+      ki[u] = kS[i * kQS + cc];
+      qi[u] = qS[i * kQS + cc];
+      l[u] = lgS[i * kQS + cc];
+    }
+    f32x4 t3 = zero4(), t4 = zero4();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float e = fast_exp(l[u] - rI);
+      t3 = __builtin_amdgcn_mfma_f32_16x16x4f32(ak[u], ki[u] * e, t3, 0, 0, 0);
+      t4 = __builtin_amdgcn_mfma_f32_16x16x4f32(aq[u], qi[u] * e, t4, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      R3[r] += (t3[r] + t4[r]) * fast_exp(rI - lgS[(16 * J + 4 * g4 + r) * kQS + cc]);
+  }
+}
+
+// The same sums with one exact exponent per pair, in the same layout (R1 and
+// R2 complete).
+__device__ __forceinline__ void pair_exact(f32x4& R1, f32x4& R2, f32x4& R3, const float* kS, const float* qS,
+                                           const float* lgS, const float* dAS, const float* dQS, int J, int cc,
+                                           int g4) {
+  const int row0 = 16 * J + 4 * g4;
+  float l[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) l[r] = lgS[(row0 + r) * kQS + cc];
+#pragma unroll 1
+  for (int j = 0; j < 16 * (J + 1); ++j) {
+    const float kj = kS[j * kQS + cc], lj = lgS[j * kQS + cc];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float ke = j <= row0 + r ? kj * fast_exp(l[r] - lj) : 0.f;
+      R1[r] += dAS[(row0 + r) * kRC + j] * ke;
+      R2[r] += dQS[(row0 + r) * kRC + j] * ke;
+    }
+  }
+#pragma unroll 1
+  for (int i = 16 * J; i < kC; ++i) {
+    const float ki = kS[i * kQS + cc], qi = qS[i * kQS + cc], x = lgS[i * kQS + cc];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float e = i >= row0 + r ? fast_exp(x - l[r]) : 0.f;
+      R3[r] += (dAS[i * kRC + row0 + r] * ki + dQS[i * kRC + row0 + r] * qi) * e;
     }
   }
 }
 
-// sm: kGradFloats floats of LDS, bS: kC more; `early` runs when the slab
-// products are done (the pair stage's input loads go out there)
-struct NoOp {
-  __device__ void operator()() const {}
-};
-template <class IT, int KP, class F = NoOp>
-__device__ __forceinline__ void grad_body(const Args<IT>& a, float* sm, float* bS, const F& early = F{}) {
-  constexpr int NT = 512;
-  constexpr int Kp = KP, CH = KP / 32;  // K-wide column tiles per wave
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, lg4 = lane >> 4;
-  const int rt = w & 3, hf = w >> 2;  // wave w: row tile rt, half hf of the column tiles
+// WHOLE: K == KP, V a multiple of the slab width and gradients aligned for
+// vector stores, so that no access needs a column test (fewer live registers:
+// the K = 128 instance spills with them); launch_all picks it.
+template <class IT, int KP, bool WHOLE>
+__global__ __launch_bounds__(kGT, kSplitOps<IT> ? 2 : 4) void grad_kernel(const Args<IT> a) {
+  using GL = GradLds<IT, KP>;
+  constexpr bool SPLIT = kSplitOps<IT>;
+  constexpr int NQ = KP / kQC;        // quarters = column tiles per wave
+  constexpr int PS = GradSlab<IT, KP, kGT>::PS;
+  __shared__ __attribute__((aligned(16))) unsigned char sm[GL::bytes];
+  __shared__ __attribute__((aligned(16))) float bS[kC];       // beta (zero past T)
+  __shared__ __attribute__((aligned(16))) float liveS[kC];    // 1, or 0 where the Vt record holds e
+  __shared__ __attribute__((aligned(16))) float dDS[KP];
+  __shared__ __attribute__((aligned(16))) float dbS[2][kC];
+  __shared__ __attribute__((aligned(16))) float tmpS[4 * kQC];
+  __shared__ __attribute__((aligned(16))) float totS[4 * kQC];  // d lg summed over each row block
+  __shared__ __attribute__((aligned(16))) float ktS[4 * kQC];   // Kt dKt summed over each row block
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g4 = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rt = w >> 1, hf = w & 1;  // row tile, parity of the column tiles
   const int64_t ch = blockIdx.x;
   const int64_t c = ch % a.NC, bh = ch / a.NC, b = bh / a.H, h = bh % a.H;
   const int64_t t0 = c * kC;
   const int Vp = a.L.Vp;
-  float* ws = a.ws + ch * a.L.per;
-  float* MS = sm + kOffM;
-  // V a multiple of the slab width: each slab's loads are issued one slab
-  // ahead, into registers; otherwise slab by slab with the edge checks.  The
-  // first slab's loads go out with beta's and N's, in one round trip.
-  const bool ahead = rows_fast(a.V, 0, Vp);
-  GradSlab<IT, KP, NT> gs;
-  if (ahead) gs.fetch(a, ws, b, t0, h, 0, tid);
-  constexpr int PN = kC * kC / 4 / NT;
-  f32x4 nv[PN];
-#pragma unroll
-  for (int it = 0; it < PN; ++it) nv[it] = *reinterpret_cast<const f32x4*>(ws + a.L.N + 4 * (tid + NT * it));
-  if (tid < kC) {
-    const int64_t t = t0 + tid;
-    bS[tid] = t < a.T ? to_float(a.beta[tok(b, t, a.T, a.H, h)]) : 0.f;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < PN; ++it) {  // M = N diag(b)
-    const int idx = 4 * (tid + NT * it);
-    *reinterpret_cast<f32x4*>(&MS[(idx >> 6) * kRC + (idx & 63)]) =
-        nv[it] * *reinterpret_cast<const f32x4*>(&bS[idx & 63]);
-  }
-
-  f32x4 aQ[CH], aT[CH], aW[CH], aA[2], aM[2];
-#pragma unroll
-  for (int m = 0; m < CH; ++m) aQ[m] = aT[m] = aW[m] = zero4();
-#pragma unroll
-  for (int m = 0; m < 2; ++m) aA[m] = aM[m] = zero4();
-  float dd = 0.f;
-  __bf16 *Ss = reinterpret_cast<__bf16*>(sm + kOffSs), *dSn = reinterpret_cast<__bf16*>(sm + kOffdSn),
-         *dOs = reinterpret_cast<__bf16*>(sm + kOffdOs), *Vts = reinterpret_cast<__bf16*>(sm + kOffVts),
-         *dVts = reinterpret_cast<__bf16*>(sm + kOffdVts), *vs = reinterpret_cast<__bf16*>(sm + kOffvs);
-  float* dVf = sm + kOffdVf;
-  const SMat mS{Ss, KP * kSR, kSR}, mdS{dSn, KP * kSR, kSR}, mdO{dOs, kC * kSR, kSR}, mVt{Vts, kC * kSR, kSR},
-      mdVt{dVts, kC * kSR, kSR}, mv{vs, kC * kSR, kSR};
-  WsTile<kC, KP, NT> kg;
-  for (int s0 = 0; s0 < Vp; s0 += kSW) {  // Vp is a multiple of the slab width
-    if (ahead) {
-      gs.store(Ss, dSn, Vts, dVts, dVf, dOs, vs, t0, a.T, tid);
-    } else {
-      if constexpr (kSplitOps<IT>) {
-        load_ws_split<KP, NT, true>(Ss, ws + a.L.S, Vp, s0, tid);
-        load_ws_split<KP, NT, true>(dSn, ws + a.L.dS, Vp, s0, tid);
-        load_ws_split<kC, NT, true>(Vts, ws + a.L.Vt, Vp, s0, tid);
-      } else {  // bf16 S, dS and Vt
-        load_ws_half<KP, NT>(Ss, ws + a.L.S, Vp, s0, tid);
-        load_ws_half<KP, NT>(dSn, ws + a.L.dS, Vp, s0, tid);
-        load_ws_half<kC, NT>(Vts, ws + a.L.Vt, Vp, s0, tid);
-      }
-      load_ws_split<kC, NT, kSplitOps<IT>>(dVts, ws + a.L.dVt, Vp, s0, tid);
-      load_ws<kC, kSW, kSS, NT>(dVf, ws + a.L.dVt, Vp, s0, tid);
-      load_rows_split<IT, NT>(dOs, a.dout, b, t0, a.T, a.H, h, a.V, s0, tid);
-      load_rows_split<IT, NT>(vs, a.v, b, t0, a.T, a.H, h, a.V, s0, tid);
-    }
-    if (ahead && s0 + kSW < Vp) gs.fetch(a, ws, b, t0, h, s0 + kSW, tid);
-    if (s0 + kSW >= Vp) kg.fetch(ws + a.L.Kg, KP, 0, tid);  // for dM += dW Kg^T after the slabs
-    __syncthreads();
-    {  // dv = M^T dVt, tile (rt, hf) of the slab
-      const f32x4 acc = mma(zero4(), Mat{MS, 1, kRC}, 16 * rt, Mat{dVf, kSS, 1}, 16 * hf, kC);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * rt + 4 * lg4 + r, col = s0 + 16 * hf + li;
-        const int64_t t = t0 + row;
-        if (t < a.T && col < a.V) a.dv[tok(b, t, a.T, a.H, h) * a.V + col] = from_compute<IT>(acc[r]);
-      }
-    }
-    // products over the slab's 32 state columns on split-bf16 operands
-#pragma unroll
-    for (int j = 0; j < CH; ++j) {
-      const int ct = hf * CH + j;
-      aQ[j] = mma3<kSplitOps<IT>>(aQ[j], mdO, 16 * rt, mS, 16 * ct, kSW);
-      aT[j] = mma3<kSplitOps<IT>>(aT[j], mVt, 16 * rt, mdS, 16 * ct, kSW);
-      aW[j] = mma3<kSplitOps<IT>>(aW[j], mdVt, 16 * rt, mS, 16 * ct, kSW);
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int ct = hf * 2 + j;
-      aA[j] = mma3<kSplitOps<IT>>(aA[j], mdO, 16 * rt, mVt, 16 * ct, kSW);
-      aM[j] = mma3<kSplitOps<IT>>(aM[j], mdVt, 16 * rt, mv, 16 * ct, kSW);
-    }
-    if (tid < Kp)
-      for (int cc = 0; cc < kSW; ++cc) {
-        float sv = static_cast<float>(Ss[tid * kSR + cc]), dv = static_cast<float>(dSn[tid * kSR + cc]);
-        if constexpr (kSplitOps<IT>) {
-          sv += static_cast<float>(Ss[KP * kSR + tid * kSR + cc]);
-          dv += static_cast<float>(dSn[KP * kSR + tid * kSR + cc]);
-        }
-        dd += dv * sv;
-      }
-    __syncthreads();
-  }
-
-  // dW = -(dVt S^T) over the slabs, Kg, and the finished dQg, dKt, dAqk, dD
-  float *X = sm + kOffX, *Y = sm + kOffY;
-#pragma unroll
-  for (int j = 0; j < CH; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * rt + 4 * lg4 + r, col = 16 * (hf * CH + j) + li;
-      X[row * kRS + col] = -aW[j][r];
-      ws[a.L.dQg + row * Kp + col] = aQ[j][r];
-      ws[a.L.dKt + row * Kp + col] = aT[j][r];
-    }
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * rt + 4 * lg4 + r, col = 16 * (hf * 2 + j) + li;
-      ws[a.L.dAqk + row * kC + col] = col <= row ? aA[j][r] : 0.f;
-    }
-  kg.template store<kRS>(Y, tid);
-  if (tid < Kp) ws[a.L.dD + tid] = dd;
-  __syncthreads();
-  early();
-  // N and A for dbeta and dA: loaded while dKg and dM are formed
-  WsTile<kC, kC, NT> wn, wa;
-  wn.fetch(ws + a.L.N, kC, 0, tid);
-  wa.fetch(ws + a.L.A, kC, 0, tid);
-#pragma unroll
-  for (int j = 0; j < CH; ++j) {  // dKg = M^T dW (this stage's products on split-bf16 operands)
-    const int ct = hf * CH + j;
-    const f32x4 acc = mma_sb(zero4(), Mat{MS, 1, kRC}, 16 * rt, Mat{X, kRS, 1}, 16 * ct, kC);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ws[a.L.dKg + (16 * rt + 4 * lg4 + r) * Kp + 16 * ct + li] = acc[r];
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j)  // dM += dW Kg^T
-    aM[j] = mma_sb(aM[j], Mat{X, kRS, 1}, 16 * rt, Mat{Y, 1, kRS}, 16 * (hf * 2 + j), Kp);
-  __syncthreads();
-
-  // dbeta and dA from N: dN = dM diag(b), T1 = N^T dN, dL = -strict(T1 N^T)
-  float *NS = sm + kOffN, *DM = sm + kOffDM, *DN = sm + kOffDN, *AS = sm + kOffA;
-  wn.template store<kRC>(NS, tid);
-  wa.template store<kRC>(AS, tid);
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * rt + 4 * lg4 + r, col = 16 * (hf * 2 + j) + li;
-      DM[row * kRC + col] = aM[j][r];
-      DN[row * kRC + col] = aM[j][r] * bS[col];
-    }
-  __syncthreads();
-  // dbeta_j = sum_i N_ij dM_ij + sum_k dL_jk A_jk: thread (j = tid / 8, p = tid % 8)
-  // takes rows i = p, p + 8, .. of the first sum and columns 8p .. 8p + 7 of
-  // the second; the eight parts of j are neighbouring lanes of one wave
-  const int bj = tid >> 3, bp = tid & 7;
-  float db = 0.f;
-#pragma unroll
-  for (int i = bp; i < kC; i += 8) db += NS[i * kRC + bj] * DM[i * kRC + bj];
-  f32x4 t1[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-    t1[j] = mma_long(zero4(), Mat{NS, 1, kRC}, 16 * rt, Mat{DN, kRC, 1}, 16 * (hf * 2 + j), kC);
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) DM[(16 * rt + 4 * lg4 + r) * kRC + 16 * (hf * 2 + j) + li] = t1[j][r];
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int ct = hf * 2 + j;
-    const f32x4 acc = mma_long(zero4(), Mat{DM, kRC, 1}, 16 * rt, Mat{NS, 1, kRC}, 16 * ct, kC);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * rt + 4 * lg4 + r, col = 16 * ct + li;
-      const float dl = col < row ? -acc[r] : 0.f;
-      DN[row * kRC + col] = dl;
-      ws[a.L.dA + row * kC + col] = bS[row] * dl;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const f32x4 x = *reinterpret_cast<const f32x4*>(&DN[bj * kRC + 8 * bp + 4 * u]);
-    const f32x4 y = *reinterpret_cast<const f32x4*>(&AS[bj * kRC + 8 * bp + 4 * u]);
-    db += x[0] * y[0] + x[1] * y[1] + x[2] * y[2] + x[3] * y[3];
-  }
-#pragma unroll
-  for (int m = 1; m < 8; m <<= 1) db += __shfl_xor(db, m);
-  if (bp == 0) {
-    const int64_t t = t0 + bj;
-    if (t < a.T) a.dbeta[tok(b, t, a.T, a.H, h)] = from_compute<IT>(db);
-  }
-}
-
-// ---- pair_body: pair sums with exact exponents and the final dq, dk, dg ------
-// Thread (column col, part p) owns rows i = p + P m of its column (P = NT / Kp,
-// RP = 64 / P rows) and forms
-//   R1_i = sum_j dA_ij k_j E_ij,  R2_i = sum_j dAqk_ij k_j E_ij   (j <= i)
-//   R3_j = sum_i dA_ij k_i E_ij,  R4_j = sum_i dAqk_ij q_i E_ij   (i >= j)
-// then dk = R1 + R3 + R4 + e^lg dKg + e^(lg_last - lg) dKt, dq = R2 + e^lg dQg,
-// d lg = k R1 - k R3 + q R2 - k R4 + Kg dKg + Qg dQg - Kt dKt (+ the last row's
-// sum(Kt dKt) + D dD), and dg as its reverse cumulative sum.
-// The sums run over blocks of 4P positions; a block only visits the owned rows
-// it can reach (a compile-time range), and a select drops the pairs on the
-// wrong side of the diagonal inside it, so no branch separates the operand
-// reads.  dA and dAqk are read four positions at a time along their rows, then
-// transposed in place for the second sum.
-// Exact path: thread (column col, part p) owns rows i = p + P m of its column.
-// Leaves d lg in qS and each thread's sum(Kt dKt) in red[p][col].
-template <class IT, int KP, int NT>
-__device__ __forceinline__ void pair_exact(const Args<IT>& a, const float* ws, float* kS, float* qS, float* lgS,
-                                           float* dAS, float* dQS, float* red, int64_t b, int64_t h, int64_t t0,
-                                           int tid) {
-  constexpr int RP = kC * KP / NT;  // rows per thread
-  constexpr int P = kC / RP;        // parts per column
-  constexpr int JB = 4 * P;         // positions per block
-  constexpr int NB = kC / JB;       // blocks
-  static_assert(RP % 4 == 0 && NB * JB == kC, "rows per thread must be a multiple of 4");
-  constexpr int Kp = KP;
-  const int col = tid % Kp, part = tid / Kp;
-  float li[RP], R1[RP], R2[RP], R3[RP], R4[RP];
-#pragma unroll
-  for (int m = 0; m < RP; ++m) {
-    li[m] = lgS[(part + P * m) * kRS + col];
-    R1[m] = R2[m] = R3[m] = R4[m] = 0.f;
-  }
-#pragma unroll
-  for (int jb = 0; jb < NB; ++jb) {  // j-sums: rows i >= j
-#pragma unroll 1
-    for (int j4 = jb * JB; j4 < (jb + 1) * JB; j4 += 4) {
-      f32x4 kj, lj;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        kj[u] = kS[(j4 + u) * kRS + col];
-        lj[u] = lgS[(j4 + u) * kRS + col];
-      }
-#pragma unroll
-      for (int m0 = 4 * jb; m0 < RP; m0 += 4) {  // four rows at a time: reads first
-        f32x4 da[4], dq[4];
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int i = part + P * (m0 + x);
-          da[x] = *reinterpret_cast<const f32x4*>(&dAS[i * kRC + j4]);
-          dq[x] = *reinterpret_cast<const f32x4*>(&dQS[i * kRC + j4]);
-        }
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int m = m0 + x, i = part + P * m;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const float e = fast_exp(li[m] - lj[u]);
-            const float ke = j4 + u <= i ? kj[u] * e : 0.f;
-            R1[m] += da[x][u] * ke;
-            R2[m] += dq[x][u] * ke;
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);  // bounds the live operands
-      }
-    }
-  }
-  __syncthreads();
-  for (int idx = tid; idx < kC * kC; idx += NT) {  // transpose dA and dAqk in place
-    const int r = idx >> 6, cc = idx & 63;
-    if (r < cc) {
-      const float x = dAS[r * kRC + cc], y = dQS[r * kRC + cc];
-      dAS[r * kRC + cc] = dAS[cc * kRC + r];
-      dQS[r * kRC + cc] = dQS[cc * kRC + r];
-      dAS[cc * kRC + r] = x;
-      dQS[cc * kRC + r] = y;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int ib = 0; ib < NB; ++ib) {  // i-sums: rows j <= i
-#pragma unroll 1
-    for (int i4 = ib * JB; i4 < (ib + 1) * JB; i4 += 4) {
-      f32x4 ki4, qi4, li4;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        ki4[u] = kS[(i4 + u) * kRS + col];
-        qi4[u] = qS[(i4 + u) * kRS + col];
-        li4[u] = lgS[(i4 + u) * kRS + col];
-      }
-#pragma unroll
-      for (int m0 = 0; m0 < 4 * (ib + 1) && m0 < RP; m0 += 4) {
-        f32x4 da[4], dq[4];
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int j = part + P * (m0 + x);
-          da[x] = *reinterpret_cast<const f32x4*>(&dAS[j * kRC + i4]);
-          dq[x] = *reinterpret_cast<const f32x4*>(&dQS[j * kRC + i4]);
-        }
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int m = m0 + x, j = part + P * m;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const float e = fast_exp(li4[u] - li[m]);
-            const float w = i4 + u >= j ? e : 0.f;
-            R3[m] += da[x][u] * ki4[u] * w;
-            R4[m] += dq[x][u] * qi4[u] * w;
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-  }
-  const float last = lgS[(kC - 1) * kRS + col];
-  __syncthreads();  // every read of q ends before d lg overwrites it
-  float lastsum = 0.f;
-  float gKg[RP], gKt[RP], gQg[RP];
-#pragma unroll
-  for (int m = 0; m < RP; ++m) {  // every load before the first store
-    const int64_t rec = static_cast<int64_t>(part + P * m) * Kp + col;
-    gKg[m] = ws[a.L.dKg + rec];
-    gKt[m] = ws[a.L.dKt + rec];
-    gQg[m] = ws[a.L.dQg + rec];
-  }
-#pragma unroll
-  for (int m = 0; m < RP; ++m) {
-    const int i = part + P * m;
-    const float kv = kS[i * kRS + col], qv = qS[i * kRS + col];
-    const float e = fast_exp(li[m]), te = fast_exp(last - li[m]);
-    const float dKg = gKg[m], dKt = gKt[m], dQg = gQg[m];
-    const float dk = R1[m] + R3[m] + R4[m] + e * dKg + te * dKt;
-    const float dq = R2[m] + e * dQg;
-    const float ktd = te * kv * dKt;
-    qS[i * kRS + col] = kv * (R1[m] - R3[m] - R4[m]) + qv * R2[m] + e * kv * dKg + e * qv * dQg - ktd;
-    lastsum += ktd;
-    const int64_t t = t0 + i;
-    if (t < a.T && col < a.K) {
-      const int64_t off = tok(b, t, a.T, a.H, h) * a.K + col;
-      a.dq[off] = from_compute<IT>(dq);
-      a.dk[off] = from_compute<IT>(dk);
-    }
-  }
-  red[part * 128 + col] = lastsum;
-}
-
-// MFMA path (NT = 512, eight waves): wave w owns rows 16J.. (J = w / 2) and
-// half of the column tiles.  With r_I = lg at row 16I and i in block I,
-//   R1_I = e^(lg - r_I) (dA_I,: (k e^(r_I - lg))),  R2 the same with dAqk,
-//   R3_J = sum_{I >= J} e^(r_I - lg) (dA_IJ^T (k e^(lg - r_I))_I),  R4 with dAqk, q.
-// Leaves d lg in qS and partial sums of Kt dKt in red[4J + g][col].
-template <class IT, int KP>
-__device__ __forceinline__ void pair_mfma(const Args<IT>& a, const float* ws, float* kS, float* qS, float* lgS,
-                                          float* dAS, float* dQS, float* red, int64_t b, int64_t h, int64_t t0,
-                                          int tid) {
-  constexpr int CW = KP / 32;  // column tiles per wave
-  const int w = tid >> 6, lane = tid & 63, li = lane & 15, lg4 = lane >> 4;
-  const int J = w >> 1, ct0 = (w & 1) * CW;
-  f32x4 R1[CW], R2[CW], R3[CW], R4[CW];
-#pragma unroll
-  for (int ct = 0; ct < CW; ++ct) R1[ct] = R2[ct] = R3[ct] = R4[ct] = zero4();
-  {  // R1, R2 over j < 16 (J + 1): the column tiles inside the reduction loop,
-     // so 2 CW independent accumulation chains keep the MFMA pipe full
-    float rI[CW];
-#pragma unroll
-    for (int ct = 0; ct < CW; ++ct) rI[ct] = lgS[16 * J * kRS + 16 * (ct0 + ct) + li];
-    for (int k0 = 0; k0 < 16 * (J + 1); k0 += 4) {
-      const int j = k0 + lg4;
-      const float ak = dAS[(16 * J + li) * kRC + j], aq = dQS[(16 * J + li) * kRC + j];
-#pragma unroll
-      for (int ct = 0; ct < CW; ++ct) {
-        const int cc = 16 * (ct0 + ct) + li;
-        const float bk = kS[j * kRS + cc] * fast_exp(rI[ct] - lgS[j * kRS + cc]);
-        R1[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(ak, bk, R1[ct], 0, 0, 0);
-        R2[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(aq, bk, R2[ct], 0, 0, 0);
-      }
-    }
-  }
-  // the element's gradient pieces from the grad kernel: their loads go out
-  // now and land while R3 and R4 are formed
-  float gKg[CW][4], gKt[CW][4], gQg[CW][4];
-#pragma unroll
-  for (int ct = 0; ct < CW; ++ct)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t rec = static_cast<int64_t>(16 * J + 4 * lg4 + r) * KP + 16 * (ct0 + ct) + li;
-      gKg[ct][r] = ws[a.L.dKg + rec];
-      gKt[ct][r] = ws[a.L.dKt + rec];
-      gQg[ct][r] = ws[a.L.dQg + rec];
-    }
-  for (int I = J; I < 4; ++I) {  // R3, R4 over rows i of block I >= J
-#pragma unroll
-    for (int ct = 0; ct < CW; ++ct) {
-      const int cc = 16 * (ct0 + ct) + li;
-      const float rI = lgS[16 * I * kRS + cc];
-      f32x4 t3 = zero4(), t4 = zero4();
-#pragma unroll
-      for (int k0 = 0; k0 < 16; k0 += 4) {
-        const int i = 16 * I + k0 + lg4;
-        const float e = fast_exp(lgS[i * kRS + cc] - rI);
-        t3 = __builtin_amdgcn_mfma_f32_16x16x4f32(dAS[i * kRC + 16 * J + li], kS[i * kRS + cc] * e, t3, 0, 0, 0);
-        t4 = __builtin_amdgcn_mfma_f32_16x16x4f32(dQS[i * kRC + 16 * J + li], qS[i * kRS + cc] * e, t4, 0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float sc = fast_exp(rI - lgS[(16 * J + 4 * lg4 + r) * kRS + cc]);
-        R3[ct][r] += t3[r] * sc;
-        R4[ct][r] += t4[r] * sc;
-      }
-    }
-  }
-  // the element's own inputs, all read before any store
-  float kv[CW][4], qv[CW][4], lv[CW][4];
-#pragma unroll
-  for (int ct = 0; ct < CW; ++ct)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * J + 4 * lg4 + r, cc = 16 * (ct0 + ct) + li;
-      kv[ct][r] = kS[row * kRS + cc];
-      qv[ct][r] = qS[row * kRS + cc];
-      lv[ct][r] = lgS[row * kRS + cc];
-    }
-  __syncthreads();  // every read of q ends before d lg overwrites it
-#pragma unroll
-  for (int ct = 0; ct < CW; ++ct) {
-    const int cc = 16 * (ct0 + ct) + li;
-    const float rJ = lgS[16 * J * kRS + cc], last = lgS[(kC - 1) * kRS + cc];
-    float part = 0.f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * J + 4 * lg4 + r;
-      const float f1 = fast_exp(lv[ct][r] - rJ);
-      const float r1 = R1[ct][r] * f1, r2 = R2[ct][r] * f1, r3 = R3[ct][r], r4 = R4[ct][r];
-      const float e = fast_exp(lv[ct][r]), te = fast_exp(last - lv[ct][r]);
-      const float k_ = kv[ct][r], q_ = qv[ct][r];
-      const float dk = r1 + r3 + r4 + e * gKg[ct][r] + te * gKt[ct][r];
-      const float dq = r2 + e * gQg[ct][r];
-      const float ktd = te * k_ * gKt[ct][r];
-      qS[row * kRS + cc] = k_ * (r1 - r3 - r4) + q_ * r2 + e * k_ * gKg[ct][r] + e * q_ * gQg[ct][r] - ktd;
-      part += ktd;
-      const int64_t t = t0 + row;
-      if (t < a.T && cc < a.K) {
-        const int64_t off = tok(b, t, a.T, a.H, h) * a.K + cc;
-        a.dq[off] = from_compute<IT>(dq);
-        a.dk[off] = from_compute<IT>(dk);
-      }
-    }
-    red[(4 * J + lg4) * 128 + cc] = part;
-  }
-}
-
-// ---- pair_body: the pair sums and the final dq, dk, dg ------------------------
-//   R1_i = sum_j dA_ij k_j E_ij,  R2_i = sum_j dAqk_ij k_j E_ij   (j <= i)
-//   R3_j = sum_i dA_ij k_i E_ij,  R4_j = sum_i dAqk_ij q_i E_ij   (i >= j)
-// then dk = R1 + R3 + R4 + e^lg dKg + e^(lg_last - lg) dKt, dq = R2 + e^lg dQg,
-// d lg = k R1 - k R3 + q R2 - k R4 + Kg dKg + Qg dQg - Kt dKt (+ the last row's
-// sum(Kt dKt) + D dD), and dg as its reverse cumulative sum.  The sums run on
-// the MFMA with the block factorisation of the decay unless the chunk needs
-// the exact pairwise path.
-// The pair kernel's LDS: k, q and lg tiles [64][kRS], dA and dAqk [64][kRC],
-// and the partial sums `red` [16][128], kPairFloats floats in this order.
-constexpr int kPairFloats = 3 * kC * kRS + 2 * kC * kRC + 16 * 128;
-// PRE: k, q and g of the chunk arrive in rk, rq, rg (fetched during the
-// gradient stage) when their rows take the whole-group path
-template <class IT, int KP, int NT, bool PRE>
-__device__ __forceinline__ void pair_body(const Args<IT>& a, float* lds, const RowTile<IT, KP, NT>& rk,
-                                          const RowTile<IT, KP, NT>& rq, const RowTile<IT, KP, NT>& rg) {
-  static_assert(NT == 512, "the MFMA path uses eight waves");
-  float *kS = lds, *qS = kS + kC * kRS, *lgS = qS + kC * kRS, *dAS = lgS + kC * kRS, *dQS = dAS + kC * kRC;
-  float* red = dQS + kC * kRC;
-  const int tid = threadIdx.x;
-  const int64_t ch = blockIdx.x;
-  const int64_t c = ch % a.NC, bh = ch / a.NC, b = bh / a.H, h = bh % a.H;
-  const int64_t t0 = c * kC;
   const float* ws = a.ws + ch * a.L.per;
+  float* NS = reinterpret_cast<float*>(sm + GL::NS);
+  __bf16* Ss = reinterpret_cast<__bf16*>(sm + GL::S);
+  __bf16* dSn = reinterpret_cast<__bf16*>(sm + GL::dS);
+  __bf16* dOs = reinterpret_cast<__bf16*>(sm + GL::dO);
+  __bf16* Vts = reinterpret_cast<__bf16*>(sm + GL::Vt);
+  __bf16* dvs = reinterpret_cast<__bf16*>(sm + GL::dv);
+  float* dVf = reinterpret_cast<float*>(sm + GL::dVf);
+  constexpr int pS = KP * kSR, pC = kC * kSR;  // lo-plane offsets
+  // the chunk's first rows as uniform bases; row offsets in 32 bits (see RowTile)
+  const int64_t tok0 = tok(b, t0, a.T, a.H, h);
+  const int rows = row_limit(t0, a.T);
+  const unsigned stepV = static_cast<unsigned>(a.H * a.V), stepK = static_cast<unsigned>(a.H * a.K);
+  const IT* dO0 = a.dout + tok0 * a.V;
+  IT* dv0 = a.dv + tok0 * a.V;
+  const bool v4 = WHOLE || (a.V & 3) == 0;
+
+  GradSlab<IT, KP, kGT> gs;
+  gs.fetch(a, ws, dO0, stepV, rows, 0, tid, WHOLE || (v4 && kSW <= a.V));
   {
-    // dA and dAqk go out first (no branch), then k, q, g: one round trip
-    constexpr int PW = kC * (kC / 4) / NT;
-    f32x4 wa[PW], wq[PW];
+    constexpr int PN = kC * kC / 4 / kGT;
+    f32x4 nv[PN];
 #pragma unroll
-    for (int it = 0; it < PW; ++it) {
-      const int item = tid + NT * it, r = item / (kC / 4), c4 = (item % (kC / 4)) * 4;
-      wa[it] = *reinterpret_cast<const f32x4*>(ws + a.L.dA + r * kC + c4);
-      wq[it] = *reinterpret_cast<const f32x4*>(ws + a.L.dAqk + r * kC + c4);
-    }
-    if (PRE && rows_fast(a.K, 0, KP)) {
-      rk.template store<kRS>(kS, t0, a.T, tid);
-      rq.template store<kRS>(qS, t0, a.T, tid);
-      rg.template store<kRS>(lgS, t0, a.T, tid);
-    } else {
-      load_kqg<IT, KP, NT>(kS, qS, lgS, a, b, t0, h, tid, a.T);
+    for (int it = 0; it < PN; ++it) nv[it] = *reinterpret_cast<const f32x4*>(ws + a.L.N + 4 * (tid + kGT * it));
+    if (tid < kC) {
+      const int64_t t = t0 + tid;
+      bS[tid] = t < a.T ? to_float(a.beta[tok(b, t, a.T, a.H, h)]) : 0.f;
+      liveS[tid] = ws[a.L.live + tid];
     }
 #pragma unroll
-    for (int it = 0; it < PW; ++it) {
-      const int item = tid + NT * it, r = item / (kC / 4), c4 = (item % (kC / 4)) * 4;
-      *reinterpret_cast<f32x4*>(&dAS[r * kRC + c4]) = wa[it];
-      *reinterpret_cast<f32x4*>(&dQS[r * kRC + c4]) = wq[it];
+    for (int it = 0; it < PN; ++it) {
+      const int idx = 4 * (tid + kGT * it);
+      *reinterpret_cast<f32x4*>(&NS[(idx >> 6) * kRC + (idx & 63)]) = nv[it];
     }
   }
-  __syncthreads();
-  const bool rising = chunk_cumsum<KP>(lgS, red, tid);  // red is written later
-  int nred;
-  if (!needs_exact<KP, NT>(lgS, rising, tid)) {
-    pair_mfma<IT, KP>(a, ws, kS, qS, lgS, dAS, dQS, red, b, h, t0, tid);
-    nred = 16;
-  } else {
-    pair_exact<IT, KP, NT>(a, ws, kS, qS, lgS, dAS, dQS, red, b, h, t0, tid);
-    nred = kC / (kC * KP / NT);
-  }
-  __syncthreads();
-  {  // dg = reverse cumulative sum of d lg, by quarters of 16 rows (totals through kS)
-    const int cc = tid % KP, p = tid / KP;
-    float v[16];
-    if (p < 4) {
+  f32x4 aQ[NQ], aT[NQ], aW[NQ], aA[2], aD[2];
 #pragma unroll
-      for (int r = 15; r >= 0; --r) v[r] = qS[(16 * p + r) * kRS + cc] + (r < 15 ? v[r + 1] : 0.f);
-      kS[p * 128 + cc] = v[0];
-    }
+  for (int j = 0; j < NQ; ++j) aQ[j] = aT[j] = aW[j] = zero4();
+#pragma unroll
+  for (int m = 0; m < 2; ++m) aA[m] = aD[m] = zero4();
+  float dd[PS], db[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int it = 0; it < PS; ++it) dd[it] = 0.f;
+  bool liveA = true, liveB[2] = {true, true};
+  QuarterTiles<IT> in;
+
+  for (int s0 = 0; s0 < Vp; s0 += kSW) {  // Vp is a multiple of the slab width
+    // per-lane addresses formed in the loop
+    const int tq = opaque(tid), li = tq & 15, g4 = (tq >> 4) & 3;
+    gs.store(Ss, dSn, Vts, dVf, dOs, dd, rows, tq);
     __syncthreads();
-    if (p < 4) {
-      float run = fast_exp(lgS[(kC - 1) * kRS + cc]) * ws[a.L.dD + cc];
-      for (int q = 0; q < nred; ++q) run += red[q * 128 + cc];
-      for (int q = p + 1; q < 4; ++q) run += kS[q * 128 + cc];
+    if (s0 == 0) {
+      liveA = liveS[16 * rt + li] != 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t t = t0 + 16 * p + r;
-        if (t < a.T && cc < a.K) a.dg[tok(b, t, a.T, a.H, h) * a.K + cc] = from_compute<IT>(v[r] + run);
+      for (int m = 0; m < 2; ++m) liveB[m] = liveS[16 * (2 * m + hf) + li] != 0.f;
+    }
+    if (s0 + kSW < Vp)
+      gs.fetch(a, ws, dO0, stepV, rows, s0 + kSW, tq, WHOLE || (v4 && s0 + 2 * kSW <= a.V));
+    // E = N^T dVt, tile (rt, hf) of the slab (N is lower triangular)
+    const f32x4 E = mma(zero4(), Mat{NS + 16 * rt * kRC, 1, kRC}, 16 * rt, Mat{dVf + 16 * rt * kSS, kSS, 1}, 16 * hf,
+                        kC - 16 * rt);
+    SlabFrag<SPLIT> fo, fv, fs, fb;
+    fo.load(dOs, pC, 16 * rt, li, g4);
+    fv.load(Vts, pC, 16 * rt, li, g4);
+    fv.keep(liveA);
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {  // dQg += dO S^T, dKt += Vt dS'^T
+      fs.load(Ss, pS, 16 * (2 * j + hf), li, g4);
+      aQ[j] = mma_frag<SPLIT>(fo, fs, aQ[j]);
+      fs.load(dSn, pS, 16 * (2 * j + hf), li, g4);
+      aT[j] = mma_frag<SPLIT>(fv, fs, aT[j]);
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {  // dAqk += dO Vt^T (blocks on and below the diagonal)
+      if (2 * m + hf <= rt) {
+        fb.load(Vts, pC, 16 * (2 * m + hf), li, g4);
+        fb.keep(liveB[m]);
+        aA[m] = mma_frag<SPLIT>(fo, fb, aA[m]);
       }
     }
-  }
-}
-
-// ---- grad_pair_kernel: grad_body, then pair_body on the same chunk ------------
-// The gradient records grad_body writes (dQg, dKt, dKg, dA, dAqk, dD: 128 KB
-// per chunk at K=V=128) are read back by pair_body in the same workgroup right
-// after, while they are still in this XCD's L2, instead of by a second kernel
-// from HBM.  The two bodies use one LDS buffer in turn.
-constexpr int kGradPairFloats = kGradFloats + kC > kPairFloats ? kGradFloats + kC : kPairFloats;
-template <class IT, int KP>
-__global__ __launch_bounds__(512) void grad_pair_kernel(const Args<IT> a) {
-  __shared__ __attribute__((aligned(16))) float lds[kGradPairFloats];
-  // single-operand inputs fetch the pair stage's k, q, g while the gradient
-  // stage forms dKg, dM, dbeta and dA (registers allow it; f32 inputs load
-  // them in the pair stage)
-  constexpr bool kPre = !kSplitOps<IT>;
-  RowTile<IT, KP, 512> rk, rq, rg;
-  const int64_t ch = blockIdx.x, c = ch % a.NC, bh = ch / a.NC, b = bh / a.H, h = bh % a.H;
-  auto early = [&] {
-    if (kPre && rows_fast(a.K, 0, KP)) {
-      rk.fetch(a.k, b, c * kC, a.T, a.H, h, a.K, 0, threadIdx.x);
-      rq.fetch(a.q, b, c * kC, a.T, a.H, h, a.K, 0, threadIdx.x);
-      rg.fetch(a.g, b, c * kC, a.T, a.H, h, a.K, 0, threadIdx.x);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * rt + 4 * g4 + r, cl = 16 * hf + li;
+      float e = static_cast<float>(Vts[row * kSR + cl]);
+      if constexpr (SPLIT) e += static_cast<float>(Vts[pC + row * kSR + cl]);
+      db[r] += E[r] * e;
+      const float dv = bS[row] * E[r];
+      __bf16 x, y;
+      split_bf16(dv, x, y);
+      dvs[row * kSR + cl] = x;
+      if constexpr (SPLIT) dvs[pC + row * kSR + cl] = y;
+      if constexpr (!__is_same(IT, bf16)) {
+        if (row < rows && (WHOLE || s0 + cl < a.V)) dv0[static_cast<unsigned>(row) * stepV + s0 + cl] = from_compute<IT>(dv);
+      }
     }
-  };
-  grad_body<IT, KP>(a, lds, lds + kGradFloats, early);
-  __syncthreads();  // every record written and every LDS read of grad_body done
-  pair_body<IT, KP, 512, kPre>(a, lds, rk, rq, rg);
+    __syncthreads();
+    fv.load(dvs, pC, 16 * rt, li, g4);
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {  // -dKg += dv S^T
+      fs.load(Ss, pS, 16 * (2 * j + hf), li, g4);
+      aW[j] = mma_frag<SPLIT>(fv, fs, aW[j]);
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m)  // -dA += dv Vt^T
+      if (2 * m + hf <= rt) {
+        fb.load(Vts, pC, 16 * (2 * m + hf), li, g4);
+        fb.keep(liveB[m]);
+        aD[m] = mma_frag<SPLIT>(fv, fb, aD[m]);
+      }
+    if constexpr (__is_same(IT, bf16)) {  // dv rounded to bf16 is the tile itself
+      const int r = tq >> 3, c4 = (tq & 7) * 4, col = s0 + c4;
+      if (r < rows) {
+        const bf16x4 x = *reinterpret_cast<const bf16x4*>(dvs + r * kSR + c4);
+        bf16* dst = dv0 + (static_cast<unsigned>(r) * stepV + static_cast<unsigned>(col));
+        if (WHOLE) {
+          *reinterpret_cast<bf16x4*>(dst) = x;
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (col + u < a.V) dst[u] = from_compute<bf16>(static_cast<float>(x[u]));
+        }
+      }
+    }
+    __syncthreads();
+  }
+
+  in.fetch(a, b, t0, h, 0, tid);  // the second stage's first quarter
+  // dA, dAqk, dD and dbeta
+  float* dAS = reinterpret_cast<float*>(sm + GL::dA);
+  float* dQS = reinterpret_cast<float*>(sm + GL::dAqk);
+  float* kS = reinterpret_cast<float*>(sm + GL::k);
+  float* qS = reinterpret_cast<float*>(sm + GL::q);
+  float* lgS = reinterpret_cast<float*>(sm + GL::lg);
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * rt + 4 * g4 + r, col = 16 * (2 * m + hf) + li;
+      dAS[row * kRC + col] = col < row ? -aD[m][r] : 0.f;
+      dQS[row * kRC + col] = col <= row ? aA[m][r] : 0.f;
+    }
+#pragma unroll
+  for (int it = 0; it < PS; ++it) {
+    float x = dd[it];
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1) x += __shfl_xor(x, m);
+    if ((tid & 7) == 0) dDS[(tid >> 3) + 64 * it] = x;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float x = db[r];
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) x += __shfl_xor(x, m);
+    if (li == 0) dbS[hf][16 * rt + 4 * g4 + r] = x;
+  }
+#pragma unroll 1
+  for (int qt = 0; qt < NQ; ++qt) {
+    const int c0 = qt * kQC, tq = opaque(tid), li = tq & 15, g4 = (tq >> 4) & 3;
+    in.store(kS, qS, lgS, a, b, t0, h, c0, tq, a.T);
+    __syncthreads();
+    if (qt == 0 && tq < kC && t0 + tq < a.T) {
+      const float s = dbS[0][tq] + dbS[1][tq];
+      a.dbeta[tok(b, t0 + tq, a.T, a.H, h)] = from_compute<IT>(liveS[tq] != 0.f ? s / bS[tq] : s);
+    }
+    if (qt + 1 < NQ) in.fetch(a, b, t0, h, c0 + kQC, tq);
+    const bool rising = chunk_cumsum<kQC, kQS>(lgS, tmpS, tq);
+    const bool exact = __syncthreads_or(rising || decay_risk<kQC, kGT, kQS>(lgS, tq));
+    const int cc = 16 * hf + li;
+    f32x4 R1 = zero4(), R2 = zero4(), R3 = zero4();
+    if (!exact)
+      pair_mfma(R1, R2, R3, kS, qS, lgS, dAS, dQS, rt, cc, li, g4);
+    else
+      pair_exact(R1, R2, R3, kS, qS, lgS, dAS, dQS, rt, cc, g4);
+    f32x4 gQ = aQ[0], gT = aT[0], gW = aW[0];
+#pragma unroll
+    for (int j = 1; j < NQ; ++j)
+      if (qt == j) gQ = aQ[j], gT = aT[j], gW = aW[j];
+    const float rJ = lgS[16 * rt * kQS + cc], last = lgS[(kC - 1) * kQS + cc];
+    float dq[4], dk[4], dl[4], ktsum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int o = (16 * rt + 4 * g4 + r) * kQS + cc;
+      const float lv = lgS[o], kv = kS[o], qv = qS[o];
+      const float f1 = exact ? 1.f : fast_exp(lv - rJ), e = fast_exp(lv), te = fast_exp(last - lv);
+      const float kt = te * gT[r];
+      const float plus = f1 * R1[r] - e * gW[r], minus = R3[r] + kt;
+      dq[r] = f1 * R2[r] + e * gQ[r];
+      dk[r] = plus + minus;
+      dl[r] = kv * (plus - minus) + qv * dq[r];
+      ktsum += kv * kt;
+    }
+    // suffix sums of d lg: over the lane's rows, the row groups, the row blocks
+#pragma unroll
+    for (int r = 2; r >= 0; --r) dl[r] += dl[r + 1];
+    float incl = dl[0];
+    {
+      const float y = __shfl_down(incl, 16);
+      incl += g4 < 3 ? y : 0.f;
+      const float z = __shfl_down(incl, 32);
+      incl += g4 < 2 ? z : 0.f;
+    }
+    float after = __shfl_down(incl, 16);
+    after = g4 < 3 ? after : 0.f;
+    ktsum += __shfl_xor(ktsum, 16);
+    ktsum += __shfl_xor(ktsum, 32);
+    if (g4 == 0) {
+      totS[rt * kQC + cc] = incl;
+      ktS[rt * kQC + cc] = ktsum;
+    }
+    __syncthreads();  // the totals are in place and every read of the tiles is done
+    after += fast_exp(last) * dDS[c0 + cc];
+#pragma unroll
+    for (int J = 0; J < 4; ++J) after += ktS[J * kQC + cc] + (J > rt ? totS[J * kQC + cc] : 0.f);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int o = (16 * rt + 4 * g4 + r) * kQS + cc;
+      qS[o] = dq[r];
+      kS[o] = dk[r];
+      lgS[o] = dl[r] + after;
+    }
+    __syncthreads();
+    {
+      const int r = tq >> 3, c4 = (tq & 7) * 4, col = c0 + c4, K = static_cast<int>(a.K);
+      if (r < rows && (WHOLE || col < K)) {
+        const unsigned off = static_cast<unsigned>(r) * stepK + static_cast<unsigned>(col);
+        put_row4<IT>(a.dq + tok0 * a.K, off, col, K, WHOLE, *reinterpret_cast<const f32x4*>(&qS[r * kQS + c4]));
+        put_row4<IT>(a.dk + tok0 * a.K, off, col, K, WHOLE, *reinterpret_cast<const f32x4*>(&kS[r * kQS + c4]));
+        put_row4<IT>(a.dg + tok0 * a.K, off, col, K, WHOLE, *reinterpret_cast<const f32x4*>(&lgS[r * kQS + c4]));
+      }
+    }
+    __syncthreads();
+  }
 }
 
 
@@ -2439,9 +2210,9 @@ using namespace kda;
 size_t chunk_bwd_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int in_dtype) {
   if (in_dtype == KDA_DTYPE_F64) return chunk_bwd_f64_workspace_bytes(B, T, H, K, V);
   // bf16 and f16 inputs keep the single-operand records (bwd::kSplitOps)
-  const bwd::Layout L = bwd::make_layout(K, V, true, in_dtype == KDA_DTYPE_F32);
+  const int64_t rec = bwd::workspace_record(K, V, in_dtype == KDA_DTYPE_F32);
   const int64_t nc = (T + bwd::kC - 1) / bwd::kC;
-  return static_cast<size_t>(B * H * nc * L.per + bwd::seg_floats(K, V, B * H, nc, 2)) * sizeof(float);
+  return static_cast<size_t>(B * H * nc * rec + bwd::seg_floats(K, V, B * H, nc, 2)) * sizeof(float);
 }
 
 size_t chunk_split_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int in_dtype) {
@@ -2507,7 +2278,8 @@ static int run_split(const IT* q, const IT* k, const IT* v, const IT* g, const I
   a.valid = valid, a.sT = sT, a.out = out;
   set_segments(a, 1);
   const int64_t chunks = B * H * a.NC;
-  if (chunks > 0x7fffffffLL || B * H * a.nseg > 0x7fffffffLL || bwd::combine_blocks(a) > 0x7fffffffLL) {
+  if (chunks > 0x7fffffffLL || B * H * a.nseg > 0x7fffffffLL || bwd::combine_blocks(a) > 0x7fffffffLL ||
+      H > bwd::kMaxHeads) {
     set_detail("chunk_fwd: grid too large");
     return KDA_ERR_UNSUPPORTED;
   }
@@ -2555,14 +2327,20 @@ template <class IT, int KP>
 static void launch_all(const bwd::Args<IT>& a, dim3 chunks, hipStream_t s) {
   hipLaunchKernelGGL((bwd::prep_kernel<IT, KP>), chunks, dim3(bwd::kPT), 0, s, a);
   launch_scans<IT, KP>(a, s);
-  hipLaunchKernelGGL((bwd::grad_pair_kernel<IT, KP>), chunks, dim3(512), 0, s, a);
+  const uintptr_t grads = reinterpret_cast<uintptr_t>(a.dq) | reinterpret_cast<uintptr_t>(a.dk) |
+                          reinterpret_cast<uintptr_t>(a.dv) | reinterpret_cast<uintptr_t>(a.dg);
+  if (a.K == KP && a.V == a.L.Vp && grads % (4 * sizeof(IT)) == 0)
+    hipLaunchKernelGGL((bwd::grad_kernel<IT, KP, true>), chunks, dim3(bwd::kGT), 0, s, a);
+  else
+    hipLaunchKernelGGL((bwd::grad_kernel<IT, KP, false>), chunks, dim3(bwd::kGT), 0, s, a);
 }
 
 template <class IT>
 static int run_bwd(bwd::Args<IT> a, hipStream_t s) {
   set_segments(a, 2);
   const int64_t chunks = a.B * a.H * a.NC;
-  if (chunks > 0x7fffffffLL || 2 * a.B * a.H * a.nseg > 0x7fffffffLL || 2 * bwd::combine_blocks(a) > 0x7fffffffLL) {
+  if (chunks > 0x7fffffffLL || 2 * a.B * a.H * a.nseg > 0x7fffffffLL || 2 * bwd::combine_blocks(a) > 0x7fffffffLL ||
+      a.H > bwd::kMaxHeads) {
     set_detail("chunk backward: grid too large");
     return KDA_ERR_UNSUPPORTED;
   }
