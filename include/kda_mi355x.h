@@ -461,6 +461,48 @@ int kda_recurrent_bwd(const void* q, const void* k, const void* v, const void* g
 int kda_cache_gather(const void* const* src, void* const* dst, const int64_t* row_bytes, int n_tensors,
                      const int64_t* index, int64_t n_src, int64_t n_out, int* status, void* stream);
 
+/*
+ * One decode step of a whole layer (KimiDeltaAttention.forward with one token,
+ * src/kda/kda.py:98-183): the projections, ShortConv + SiLU (+ L2 norm), decay and beta
+ * gates, the recurrence step, RMSNorm x output gate and the output projection, in three
+ * launches.  Every tensor is contiguous and 16-byte aligned, in `dtype` (bf16 or f16)
+ * unless stated; linear weights are [out, in], ShortConv weights [channels, taps] in lag
+ * order; biases and norm_weight may be NULL.  key_dim and value_dim 64 or 128, d_model a
+ * multiple of 64, rank a multiple of 8 up to 256, taps up to 8.
+ *   x                : [batch, d_model];  out : [batch, out_dim]
+ *   q_hist .. v_hist : [batch, taps - 1, channels] or NULL (zeros); *_hist_out the next ones
+ *   state_in         : f32 [batch, heads, key_dim, value_dim] or NULL (zeros); state_out may
+ *                      be state_in
+ *   offset_in        : int64 [batch] or NULL (zeros); offset_out = offset_in + 1
+ *   norm_per_head    : norm_weight is [heads, value_dim] (1) or [value_dim] (0)
+ *   workspace        : kda_layer_decode_workspace_bytes(args)
+ */
+typedef struct {
+  const void* x;
+  const void *q_proj, *k_proj, *v_proj, *beta_proj, *alpha_down, *gate_proj, *alpha_up, *output_proj;
+  const void *q_bias, *k_bias, *v_bias, *beta_bias, *gate_bias, *output_bias;
+  const void *q_conv, *k_conv, *v_conv, *q_conv_bias, *k_conv_bias, *v_conv_bias;
+  const void* b_alpha;
+  const float* a_log;
+  const void* norm_weight;
+  const void *q_hist, *k_hist, *v_hist;
+  const float* state_in;
+  const int64_t* offset_in;
+  void *q_hist_out, *k_hist_out, *v_hist_out;
+  float* state_out;
+  int64_t* offset_out;
+  void* out;
+  void* workspace;
+  size_t workspace_bytes;
+  int64_t batch, d_model, out_dim, heads, key_dim, value_dim, taps, rank;
+  double g_min, eps;
+  int dtype, norm_per_head;
+} kda_layer_decode_args;
+
+size_t kda_layer_decode_workspace_bytes(const kda_layer_decode_args* args);
+
+int kda_layer_decode(const kda_layer_decode_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

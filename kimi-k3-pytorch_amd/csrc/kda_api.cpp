@@ -594,4 +594,35 @@ int kda_recurrent_bwd(const void* q, const void* k, const void* v, const void* g
                               workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
+size_t kda_layer_decode_workspace_bytes(const kda_layer_decode_args* args) {
+  if (!args || args->batch <= 0 || args->heads <= 0 || args->key_dim <= 0 || args->value_dim <= 0 || args->rank <= 0)
+    return 0;
+  return layer_decode_workspace_bytes(*args);
+}
+
+int kda_layer_decode(const kda_layer_decode_args* args, void* stream) {
+  g_detail[0] = '\0';
+  if (!args || args->batch <= 0 || args->d_model <= 0 || args->out_dim <= 0 || args->heads <= 0 ||
+      args->key_dim <= 0 || args->value_dim <= 0 || args->rank <= 0 || args->taps <= 0) {
+    set_detail("layer_decode: sizes must be positive");
+    return KDA_ERR_INVALID_ARGUMENT;
+  }
+  const kda_layer_decode_args& d = *args;
+  const bool hists = d.taps == 1 || (d.q_hist_out && d.k_hist_out && d.v_hist_out);
+  if (!d.x || !d.q_proj || !d.k_proj || !d.v_proj || !d.beta_proj || !d.alpha_down || !d.gate_proj || !d.alpha_up ||
+      !d.output_proj || !d.q_conv || !d.k_conv || !d.v_conv || !d.b_alpha || !d.a_log || !d.state_out || !d.offset_out ||
+      !d.out || !d.workspace || !hists) {
+    set_detail("layer_decode: x, the weights, the outputs and the workspace must be non-null");
+    return KDA_ERR_INVALID_ARGUMENT;
+  }
+  const void* vectors[] = {d.x,        d.q_proj,      d.k_proj,   d.v_proj,   d.beta_proj, d.alpha_down,
+                           d.gate_proj, d.output_proj, d.alpha_up, d.state_in, d.state_out, d.workspace};
+  for (const void* p : vectors)
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) {
+      set_detail("layer_decode: x, the linear weights, the states and the workspace must be 16-byte aligned");
+      return KDA_ERR_INVALID_ARGUMENT;
+    }
+  return launch_layer_decode(d, static_cast<hipStream_t>(stream));
+}
+
 }  // extern "C"

@@ -32,6 +32,25 @@ DTYPE_CODES = {
     torch.float64: 3,
 }
 
+
+class LayerDecodeArgs(ctypes.Structure):
+    """kda_layer_decode_args, field for field."""
+
+    _fields_ = (
+        [(name, ctypes.c_void_p) for name in (
+            "x", "q_proj", "k_proj", "v_proj", "beta_proj", "alpha_down", "gate_proj", "alpha_up", "output_proj",
+            "q_bias", "k_bias", "v_bias", "beta_bias", "gate_bias", "output_bias", "q_conv", "k_conv", "v_conv",
+            "q_conv_bias", "k_conv_bias", "v_conv_bias", "b_alpha", "a_log", "norm_weight", "q_hist", "k_hist",
+            "v_hist", "state_in", "offset_in", "q_hist_out", "k_hist_out", "v_hist_out", "state_out", "offset_out",
+            "out", "workspace")]
+        + [("workspace_bytes", ctypes.c_size_t)]
+        + [(name, ctypes.c_int64) for name in ("batch", "d_model", "out_dim", "heads", "key_dim", "value_dim", "taps",
+                                               "rank")]
+        + [("g_min", ctypes.c_double), ("eps", ctypes.c_double), ("dtype", ctypes.c_int),
+           ("norm_per_head", ctypes.c_int)]
+    )
+
+
 # Every exported symbol with (restype, argtypes); include/kda_mi355x.h is the source of truth.
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -90,6 +109,8 @@ SIGNATURES = {
     "kda_cache_gather": (_I, [_P, _P, _P, _I, _P, _L, _L, _P, _P]),
     "kda_recurrent_bwd_workspace_bytes": (_S, [_L, _L, _L, _L, _I]),
     "kda_recurrent_bwd": (_I, [_P] * 16 + [_L] * 5 + [_I, _P, _S, _P]),
+    "kda_layer_decode_workspace_bytes": (_S, [_P]),
+    "kda_layer_decode": (_I, [_P, _P]),
 }
 
 _lock = threading.Lock()

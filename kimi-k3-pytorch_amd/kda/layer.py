@@ -20,22 +20,25 @@ output gate (kda.py:153-161) and the ``KDAState`` handed to the next call
   projection), the output projection, and the mask.
 
 The projection GEMMs are torch's; everything between them runs in this
-library's HIP kernels.  Weights are plain tensors (``KDALayerWeights``), so a
+library's HIP kernels.  A decode step of up to ``DECODE_STEP_BATCH`` sequences
+outside autograd runs projections and all in three launches
+(``kda_layer_decode``), with the same roundings between the stages.  Weights are plain tensors (``KDALayerWeights``), so a
 reference module's parameters can be handed over with ``from_module``.
 """
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import Literal
 
 import torch
 import torch.nn.functional as F
 
-from . import fused
+from . import _lib, _prep, fused
 from .chunkwise import chunkwise_kda
 from .recurrent import recurrent_kda
-from .state import KDAState
+from .state import KDAState, ShortConvState
 from .utils import validate_attention_mask
 
 
@@ -146,6 +149,85 @@ def _validate_state(w: KDALayerWeights, hidden_states: torch.Tensor, state: KDAS
         raise ValueError("state and hidden_states must be on the same device")
 
 
+# Largest batch the native decode step takes.  Measured per call at d_model 2048
+# (16 heads x 128, bf16), native against the composed stages: 1 sequence 36 and
+# 301 us (both bound by the host), 32 45 and 293, 128 124 and 294, 256 224 and
+# 274; its projections read the weights again for every 64 sequences, so past
+# 256 the library's GEMMs are the better ones.
+DECODE_STEP_BATCH = 256
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _decode_step(w: KDALayerWeights, x: torch.Tensor, state: KDAState | None, in_place: bool) -> KDALayerOutput | None:
+    """One token per sequence through ``kda_layer_decode``, or None when the call
+    needs the composed stages: tensors that require grad, autocast, tensor
+    subclasses, layouts, dtypes or sizes the kernels do not take, or anything
+    the stages would refuse (so that they raise their own errors)."""
+    batch, H, K, V = x.shape[0], w.num_heads, w.key_head_dim, w.value_head_dim
+    dtype, device = x.dtype, x.device
+    if (batch > DECODE_STEP_BATCH or dtype not in (torch.bfloat16, torch.float16) or device.type != "cuda"
+            or K not in (64, 128) or V not in (64, 128) or not w.accumulate_state_in_fp32
+            or torch.is_autocast_enabled("cuda") or not w.eps > 0 or not w.g_min < 0):
+        return None
+    if any(t.ndim != 2 for t in (w.q_conv, w.alpha_down, w.output_proj)):
+        return None
+    d_model, kw, vw, taps = x.shape[2], H * K, H * V, w.q_conv.shape[1]
+    rank, out_dim = w.alpha_down.shape[0], w.output_proj.shape[0]
+    norm = w.norm_weight
+    per_head = norm is not None and norm.ndim == 2
+    if (d_model % 64 or d_model != vw or not 1 <= taps <= 8 or rank % 8 or not 8 <= rank <= 256
+            or w.a_log.dtype != torch.float32):
+        return None
+    hist = (batch, taps - 1)
+    expected = [
+        (x, (batch, 1, d_model)), (w.q_proj, (kw, d_model)), (w.k_proj, (kw, d_model)), (w.v_proj, (vw, d_model)),
+        (w.beta_proj, (H, d_model)), (w.alpha_down, (rank, d_model)), (w.gate_proj, (vw, d_model)),
+        (w.alpha_up, (kw, rank)), (w.output_proj, (out_dim, vw)), (w.q_proj_bias, (kw,)), (w.k_proj_bias, (kw,)),
+        (w.v_proj_bias, (vw,)), (w.beta_bias, (H,)), (w.gate_bias, (vw,)), (w.output_bias, (out_dim,)),
+        (w.q_conv, (kw, taps)), (w.k_conv, (kw, taps)), (w.v_conv, (vw, taps)), (w.q_conv_bias, (kw,)),
+        (w.k_conv_bias, (kw,)), (w.v_conv_bias, (vw,)), (w.b_alpha, (H, K)), (w.a_log, (H,)),
+        (norm, (H, V) if per_head else (V,)),
+    ]
+    buffers = (None, None, None)
+    recurrent = offset = None
+    if state is not None:
+        recurrent, offset = state.recurrent_state, state.sequence_offset
+        if recurrent.dtype != torch.float32 or offset.device != device:
+            return None
+        buffers = (state.q_conv_state.buffer, state.k_conv_state.buffer, state.v_conv_state.buffer)
+        expected += [(buffers[0], (*hist, kw)), (buffers[1], (*hist, kw)), (buffers[2], (*hist, vw)),
+                     (recurrent, (batch, H, K, V)), (offset, (batch,))]
+    grad = torch.is_grad_enabled()
+    for t, shape in expected:
+        if t is not None and (
+                type(t) not in _PLAIN or t.shape != shape or t.device != device or not t.is_contiguous()
+                or (grad and t.requires_grad)
+                or (t.dtype != dtype and t is not w.a_log and t is not recurrent and t is not offset)):
+            return None
+    ptr = [None if t is None else t.data_ptr() for t, _ in expected] + [None] * (29 - len(expected))
+    if any(p is not None and p & 15 for p in (*ptr[:9], ptr[27])):
+        return None
+    lib = _lib.load()
+    new = x.new_empty
+    outs = [new(*hist, kw), new(*hist, kw), new(*hist, vw)]
+    state_out = recurrent if in_place and recurrent is not None else new(batch, H, K, V, dtype=torch.float32)
+    offset_out = new(batch, dtype=torch.long)
+    out = new(batch, 1, out_dim)
+    args = _lib.LayerDecodeArgs(
+        *ptr, *(t.data_ptr() for t in outs), state_out.data_ptr(), offset_out.data_ptr(), out.data_ptr(), None, 0,
+        batch, d_model, out_dim, H, K, V, taps, rank, float(w.g_min), float(w.eps), _lib.dtype_code(dtype),
+        1 if per_head else 0)
+    ref = ctypes.addressof(args)
+    args.workspace_bytes = lib.kda_layer_decode_workspace_bytes(ref)
+    workspace = _prep.workspace(args.workspace_bytes, device, "kda_attention_forward's decode step")
+    args.workspace = workspace.data_ptr()
+    _lib.check(lib.kda_layer_decode(ref, _prep.stream(device)))
+    return KDALayerOutput(hidden_states=out, state=KDAState(
+        recurrent_state=state_out, q_conv_state=ShortConvState(outs[0]), k_conv_state=ShortConvState(outs[1]),
+        v_conv_state=ShortConvState(outs[2]), sequence_offset=offset_out))
+
+
 def kda_attention_forward(
     w: KDALayerWeights,
     hidden_states: torch.Tensor,
@@ -171,6 +253,10 @@ def kda_attention_forward(
     validate_attention_mask(attention_mask, batch, tokens)
     _validate_state(w, hidden_states, state)
     x = hidden_states
+    if mode == "decode" and attention_mask is None:
+        step = _decode_step(w, x, state, update_state_in_place)
+        if step is not None:
+            return step
     H, K, V = w.num_heads, w.key_head_dim, w.value_head_dim
     return_state = output_final_state or mode == "decode"
 
