@@ -462,6 +462,13 @@ int kda_cache_gather(const void* const* src, void* const* dst, const int64_t* ro
                      const int64_t* index, int64_t n_src, int64_t n_out, int* status, void* stream);
 
 /*
+ * Right-padding mask -> valid lengths (the checks of src/kda/utils.py:8-29 in one launch).
+ *   mask    : [batch, tokens] one byte per token, non-zero where valid
+ *   lengths : int32 [batch]: the row's valid tokens, or -1 when they are no prefix of the row
+ */
+int kda_mask_lengths(const uint8_t* mask, int64_t batch, int64_t tokens, int32_t* lengths, void* stream);
+
+/*
  * One decode step of a whole layer (KimiDeltaAttention.forward with one token,
  * src/kda/kda.py:98-183): the projections, ShortConv + SiLU (+ L2 norm), decay and beta
  * gates, the recurrence step, RMSNorm x output gate and the output projection, in three

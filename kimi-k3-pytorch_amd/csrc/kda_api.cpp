@@ -594,6 +594,15 @@ int kda_recurrent_bwd(const void* q, const void* k, const void* v, const void* g
                               workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
+int kda_mask_lengths(const uint8_t* mask, int64_t batch, int64_t tokens, int32_t* lengths, void* stream) {
+  g_detail[0] = '\0';
+  if (!mask || !lengths || batch <= 0 || batch > 0x7fffffffLL || tokens <= 0 || tokens > 0x7fffffffLL) {
+    set_detail("mask_lengths: mask and lengths must be non-null, batch and tokens in 1..2^31-1");
+    return KDA_ERR_INVALID_ARGUMENT;
+  }
+  return launch_mask_lengths(mask, batch, tokens, lengths, static_cast<hipStream_t>(stream));
+}
+
 size_t kda_layer_decode_workspace_bytes(const kda_layer_decode_args* args) {
   if (!args || args->batch <= 0 || args->heads <= 0 || args->key_dim <= 0 || args->value_dim <= 0 || args->rank <= 0)
     return 0;

@@ -155,6 +155,9 @@ int launch_rmsnorm_gate_bwd(const void* x, const void* w, int w_per_head, const 
 int launch_cache_gather(const void* const* src, void* const* dst, const int64_t* row_bytes, int n_tensors,
                         const int64_t* index, int64_t n_src, int64_t n_out, int* status, hipStream_t stream);
 
+// Valid lengths of a right-padding mask, -1 for other rows (csrc/kda_mask.hip).
+int launch_mask_lengths(const uint8_t* mask, int64_t batch, int64_t tokens, int32_t* lengths, hipStream_t stream);
+
 // One decode step of a layer (csrc/kda_layer_decode.hip).
 size_t layer_decode_workspace_bytes(const kda_layer_decode_args& d);
 

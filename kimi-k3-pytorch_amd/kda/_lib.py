@@ -109,6 +109,7 @@ SIGNATURES = {
     "kda_cache_gather": (_I, [_P, _P, _P, _I, _P, _L, _L, _P, _P]),
     "kda_recurrent_bwd_workspace_bytes": (_S, [_L, _L, _L, _L, _I]),
     "kda_recurrent_bwd": (_I, [_P] * 16 + [_L] * 5 + [_I, _P, _S, _P]),
+    "kda_mask_lengths": (_I, [_P, _L, _L, _P, _P]),
     "kda_layer_decode_workspace_bytes": (_S, [_P]),
     "kda_layer_decode": (_I, [_P, _P]),
 }

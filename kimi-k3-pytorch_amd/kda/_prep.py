@@ -56,13 +56,6 @@ def kernel_inputs(q, k, v, g, beta, work_dtype: torch.dtype):
     return out, kernel_dtype, arith
 
 
-def valid_lengths(attention_mask: torch.Tensor | None, device: torch.device) -> torch.Tensor | None:
-    """Monotone right-padding mask -> int32 valid length per row."""
-    if attention_mask is None:
-        return None
-    return attention_mask.to(device=device).sum(dim=1, dtype=torch.int32).contiguous()
-
-
 def state_arg(initial_state: torch.Tensor | None, arith: torch.dtype,
               work_dtype: torch.dtype | None = None) -> torch.Tensor | None:
     """The initial state in the kernels' arithmetic type.  The reference starts

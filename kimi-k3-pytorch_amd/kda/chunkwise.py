@@ -42,7 +42,7 @@ import torch
 
 from . import _lib, _prep
 from .recurrent import KDAOperatorOutput
-from .utils import accumulation_dtype, validate_core_inputs, validate_cu_seqlens
+from .utils import accumulation_dtype, checked_lengths, validate_core_inputs, validate_cu_seqlens
 
 
 def chunkwise_kda(
@@ -70,16 +70,22 @@ def chunkwise_kda(
         offsets = validate_cu_seqlens(cu_seqlens, q.shape[0] if q.ndim == 4 else -1,
                                       q.shape[1] if q.ndim == 4 else -1, attention_mask)
     num_states = None if offsets is None else len(offsets) - 1
-    batch, tokens, heads, key_dim, value_dim = validate_core_inputs(
-        q, k, v, g, beta, initial_state, attention_mask, num_states=num_states
-    )
+    batch, tokens, *_ = validate_core_inputs(q, k, v, g, beta, initial_state, None, num_states=num_states)
+    valid = checked_lengths(attention_mask, batch, tokens, q.device)
+    return checked_chunkwise(q, k, v, g, beta, initial_state, output_final_state, attention_mask, valid,
+                             accumulate_state_in_fp32, offsets)
+
+
+def checked_chunkwise(q, k, v, g, beta, initial_state, output_final_state, attention_mask, valid,
+                      accumulate_state_in_fp32, offsets=None) -> KDAOperatorOutput:
+    """``chunkwise_kda`` on checked inputs; ``valid``: the mask's int32 lengths."""
     _lib.require_gpu(q)
     work_dtype = accumulation_dtype(v.dtype, accumulate_state_in_fp32)
     if needs_grad(q, k, v, g, beta, initial_state):
         return differentiable(q, k, v, g, beta, initial_state, output_final_state, attention_mask, work_dtype,
                               recurrent=False, offsets=offsets)
-    return _forward(q, k, v, g, beta, initial_state, output_final_state, attention_mask, work_dtype, offsets,
-                    batch, tokens, heads, key_dim, value_dim)
+    return _forward(q, k, v, g, beta, initial_state, output_final_state, valid, work_dtype, offsets, *q.shape,
+                    v.shape[-1])
 
 
 # Most bytes one kernel call may take as workspace before its heads run in
@@ -89,7 +95,7 @@ def chunkwise_kda(
 WORKSPACE_LIMIT = 4 << 30
 
 
-def _forward(q, k, v, g, beta, initial_state, output_final_state, attention_mask, work_dtype, offsets,
+def _forward(q, k, v, g, beta, initial_state, output_final_state, valid, work_dtype, offsets,
              batch, tokens, heads, key_dim, value_dim) -> KDAOperatorOutput:
     lib = _lib.load()
     (qc, kc, vc, gc, bc), kernel_dtype, arith = _prep.kernel_inputs(q, k, v, g, beta, work_dtype)
@@ -97,7 +103,7 @@ def _forward(q, k, v, g, beta, initial_state, output_final_state, attention_mask
         # the chunk kernels hold at most 128 key channels per state: the exact
         # token recurrence runs instead (f64 inputs take it by design)
         warnings.warn(f"chunkwise_kda: key_dim {key_dim} > 128 runs the token-by-token recurrence kernel, "
-                      "not the chunk-parallel path (much slower on long sequences)", RuntimeWarning, stacklevel=3)
+                      "not the chunk-parallel path (much slower on long sequences)", RuntimeWarning, stacklevel=4)
     device = q.device
     n_seq = batch if offsets is None else len(offsets) - 1
     total = batch * tokens
@@ -109,7 +115,6 @@ def _forward(q, k, v, g, beta, initial_state, output_final_state, attention_mask
     )
     out = torch.empty(batch, tokens, heads, value_dim, dtype=kernel_dtype, device=device)
     cu = None if offsets is None else _prep.cu_tensor(offsets, device)
-    valid = _prep.valid_lengths(attention_mask, device)
     code = _lib.dtype_code(kernel_dtype)
     # packed documents: the longest document's length is the schedule's hint
     longest = _prep.longest_document(offsets)

@@ -29,7 +29,7 @@ import torch
 
 from . import _lib, _prep
 from .state import ShortConvState
-from .utils import validate_attention_mask
+from .utils import checked_lengths
 
 _DTYPES = (torch.float32, torch.float16, torch.bfloat16, torch.float64)
 
@@ -88,6 +88,19 @@ def conv_silu(
     when ``num_heads`` is given (``[B,T,C]`` otherwise) and the next state when
     ``output_final_state``.
     """
+    _check_conv(x, weight, bias, state, num_heads, normalize, eps)
+    valid = checked_lengths(attention_mask, x.shape[0], x.shape[1], x.device)
+    return _conv_silu(x, weight, bias, state, valid, num_heads, normalize, eps, output_final_state)
+
+
+def conv_silu_with_lengths(x, weight, bias, state, valid, *, num_heads, normalize, eps, output_final_state):
+    """``conv_silu`` for a caller that has checked its mask: ``valid`` are the
+    mask's int32 lengths (None without one)."""
+    _check_conv(x, weight, bias, state, num_heads, normalize, eps)
+    return _conv_silu(x, weight, bias, state, valid, num_heads, normalize, eps, output_final_state)
+
+
+def _check_conv(x, weight, bias, state, num_heads, normalize, eps) -> None:
     if x.ndim != 3:
         raise ValueError(f"x must have shape [B,T,C], got {tuple(x.shape)}")
     batch, tokens, channels = x.shape
@@ -117,11 +130,13 @@ def conv_silu(
         raise ValueError("normalize needs num_heads")
     if eps <= 0:
         raise ValueError("eps must be > 0")
-    validate_attention_mask(attention_mask, batch, tokens)
+
+
+def _conv_silu(x, weight, bias, state, valid, num_heads, normalize, eps, output_final_state):
     _lib.require_gpu(x)
+    batch, tokens, channels = x.shape
     head_dim = channels // num_heads if num_heads is not None else channels
     hist = None if state is None else state.buffer
-    valid = _prep.valid_lengths(attention_mask, x.device)
     cfg = (head_dim, bool(normalize), float(eps), bool(output_final_state))
     if _needs_grad(x, weight, bias, hist):
         y, hist_out = _ConvSilu.apply(x, weight, bias, hist, valid, cfg)
@@ -304,29 +319,68 @@ class _Decay(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, dg, dalpha):
         logits, a_log, bias = ctx.saved_tensors
-        lib = _lib.load()
-        batch, tokens, heads, key_dim = logits.shape
-        z = _aligned(logits)
-        zb = None if bias is None else _aligned(bias.to(logits.dtype))
-        al = a_log.to(torch.float32).contiguous()
-        if dg is None:
-            dg = torch.zeros_like(z)
-        dgc = _aligned(dg.to(z.dtype))
-        dac = None if dalpha is None else _aligned(dalpha.to(z.dtype))
-        dz = torch.empty_like(z)
-        acc = _acc_dtype(z.dtype)
-        dzb = torch.zeros(heads, key_dim, dtype=acc, device=z.device) if bias is not None and ctx.needs_input_grad[2] \
-            else None
-        dal = torch.zeros(heads, dtype=acc, device=z.device) if ctx.needs_input_grad[1] else None
-        if dzb is not None or dal is not None:
-            _alert_nondeterministic("the decay gate backward (kda_gates_bwd)")
-        _lib.check(lib.kda_gates_bwd(
-            z.data_ptr(), _lib.ptr(zb), al.data_ptr(), ctx.g_min, dgc.data_ptr(), _lib.ptr(dac), dz.data_ptr(),
-            _lib.ptr(dzb), _lib.ptr(dal), None, None, None, batch * tokens, heads, key_dim,
-            _lib.dtype_code(z.dtype), _prep.stream(z.device),
-        ))
-        return (dz if ctx.needs_input_grad[0] else None, None if dal is None else dal.to(a_log.dtype),
-                None if dzb is None else dzb.to(bias.dtype), None)
+        return (*_decay_gradients(ctx, logits, a_log, bias, dg, dalpha), None)
+
+
+def _decay_gradients(ctx, logits, a_log, bias, dg, dalpha):
+    """Gradients of the decay's logits, A_log and bias (ctx's first three inputs)."""
+    lib = _lib.load()
+    batch, tokens, heads, key_dim = logits.shape
+    z = _aligned(logits)
+    zb = None if bias is None else _aligned(bias.to(logits.dtype))
+    al = a_log.to(torch.float32).contiguous()
+    if dg is None:
+        dg = torch.zeros_like(z)
+    dgc = _aligned(dg.to(z.dtype))
+    dac = None if dalpha is None else _aligned(dalpha.to(z.dtype))
+    dz = torch.empty_like(z)
+    acc = _acc_dtype(z.dtype)
+    dzb = torch.zeros(heads, key_dim, dtype=acc, device=z.device) if bias is not None and ctx.needs_input_grad[2] \
+        else None
+    dal = torch.zeros(heads, dtype=acc, device=z.device) if ctx.needs_input_grad[1] else None
+    if dzb is not None or dal is not None:
+        _alert_nondeterministic("the decay gate backward (kda_gates_bwd)")
+    _lib.check(lib.kda_gates_bwd(
+        z.data_ptr(), _lib.ptr(zb), al.data_ptr(), ctx.g_min, dgc.data_ptr(), _lib.ptr(dac), dz.data_ptr(),
+        _lib.ptr(dzb), _lib.ptr(dal), None, None, None, batch * tokens, heads, key_dim,
+        _lib.dtype_code(z.dtype), _prep.stream(z.device),
+    ))
+    return (dz if ctx.needs_input_grad[0] else None, None if dal is None else dal.to(a_log.dtype),
+            None if dzb is None else dzb.to(bias.dtype))
+
+
+def layer_gates(decay_logits, a_log, g_min, bias, beta_logits):
+    """``(lower_bounded_decay(decay_logits, ...)[0], beta_gate(beta_logits))`` in
+    one launch each way, without the exp(g) that the operator does not read:
+    its 33 MB per 8192 tokens of 2048 channels are neither written nor, as a
+    zero gradient, read back."""
+    if decay_logits.dtype != beta_logits.dtype or decay_logits.device != beta_logits.device:
+        return lower_bounded_decay(decay_logits, a_log, g_min, bias=bias)[0], beta_gate(beta_logits)
+    if _needs_grad(decay_logits, a_log, bias, beta_logits):
+        return _LayerGates.apply(decay_logits, a_log, bias, beta_logits, float(g_min))
+    g, _, beta = _gates(decay_logits, a_log, g_min, bias, beta_logits, False)
+    return g, beta
+
+
+class _LayerGates(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, logits, a_log, bias, beta_logits, g_min):
+        g, _, beta = _gates(logits, a_log, g_min, bias, beta_logits, False)
+        ctx.save_for_backward(logits, a_log, bias, beta_logits)
+        ctx.g_min = g_min
+        ctx.set_materialize_grads(False)
+        return g, beta
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dg, dbeta):
+        logits, a_log, bias, beta_logits = ctx.saved_tensors
+        dz = dal = dzb = dl = None
+        if dg is not None:
+            dz, dal, dzb = _decay_gradients(ctx, logits, a_log, bias, dg, None)
+        if dbeta is not None and ctx.needs_input_grad[3]:
+            dl = _beta_gradient(beta_logits, dbeta)
+        return dz, dal, dzb, dl, None
 
 
 class _Beta(torch.autograd.Function):
@@ -340,15 +394,19 @@ class _Beta(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, dbeta):
         (logits,) = ctx.saved_tensors
-        lib = _lib.load()
-        bl = logits.contiguous()
-        db = dbeta.to(bl.dtype).contiguous()
-        dl = torch.empty_like(bl)
-        _lib.check(lib.kda_gates_bwd(
-            None, None, None, -1.0, None, None, None, None, None, bl.data_ptr(), db.data_ptr(), dl.data_ptr(),
-            1, bl.numel(), 1, _lib.dtype_code(bl.dtype), _prep.stream(bl.device),
-        ))
-        return dl
+        return _beta_gradient(logits, dbeta)
+
+
+def _beta_gradient(logits, dbeta):
+    lib = _lib.load()
+    bl = logits.contiguous()
+    db = dbeta.to(bl.dtype).contiguous()
+    dl = torch.empty_like(bl)
+    _lib.check(lib.kda_gates_bwd(
+        None, None, None, -1.0, None, None, None, None, None, bl.data_ptr(), db.data_ptr(), dl.data_ptr(),
+        1, bl.numel(), 1, _lib.dtype_code(bl.dtype), _prep.stream(bl.device),
+    ))
+    return dl
 
 
 def chunkwise_kda_with_decay(
@@ -374,7 +432,7 @@ def chunkwise_kda_with_decay(
     composition bit for bit.  Shapes off the MFMA path (K above 128 or not a
     multiple of 16, V not a multiple of 16 in 16..256, f32/f64 inputs) and calls under autograd run the
     two steps (both in HIP kernels); so does f16/bf16 work without an f32 state."""
-    from .chunkwise import chunkwise_kda, needs_grad
+    from .chunkwise import checked_chunkwise, needs_grad
     from .recurrent import KDAOperatorOutput
     from .utils import accumulation_dtype, validate_core_inputs, validate_cu_seqlens
 
@@ -384,7 +442,8 @@ def chunkwise_kda_with_decay(
                                       q.shape[1] if q.ndim == 4 else -1, attention_mask)
     num_states = None if offsets is None else len(offsets) - 1
     batch, tokens, heads, key_dim, value_dim = validate_core_inputs(
-        q, k, v, decay_logits, beta, initial_state, attention_mask, num_states=num_states)
+        q, k, v, decay_logits, beta, initial_state, None, num_states=num_states)
+    valid = checked_lengths(attention_mask, batch, tokens, q.device)
     _lib.require_gpu(q)
     if a_log.shape != (heads,):
         raise ValueError(f"A_log must have shape [{heads}], got {tuple(a_log.shape)}")
@@ -399,8 +458,8 @@ def chunkwise_kda_with_decay(
                 and not needs_grad(q, k, v, decay_logits, beta, initial_state, a_log, decay_bias))
     if not fused_ok:
         g, _ = lower_bounded_decay(decay_logits, a_log, g_min, bias=decay_bias)
-        return chunkwise_kda(q, k, v, g, beta, initial_state, output_final_state, attention_mask,
-                             accumulate_state_in_fp32=accumulate_state_in_fp32, cu_seqlens=cu_seqlens)
+        return checked_chunkwise(q, k, v, g, beta, initial_state, output_final_state, attention_mask, valid,
+                                 accumulate_state_in_fp32, offsets)
     lib = _lib.load()
     device = q.device
     qc, kc, vc, zc, bc = (t.contiguous() for t in (q, k, v, decay_logits, beta))
@@ -413,7 +472,6 @@ def chunkwise_kda_with_decay(
              if output_final_state else None)
     out = torch.empty(batch, tokens, heads, value_dim, dtype=q.dtype, device=device)
     cu = None if offsets is None else _prep.cu_tensor(offsets, device)
-    valid = _prep.valid_lengths(attention_mask, device)
     code = _lib.dtype_code(q.dtype)
     longest = _prep.longest_document(offsets)
     ws_bytes = lib.kda_chunk_fwd_workspace_bytes(n_seq, total, longest, heads, key_dim, value_dim, code)

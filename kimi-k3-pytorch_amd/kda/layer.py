@@ -11,11 +11,10 @@ output gate (kda.py:153-161) and the ``KDAState`` handed to the next call
 * q, k, v: the projection GEMM (``torch.nn.functional.linear``, as the
   reference's ``nn.Linear``), then ``fused.conv_silu`` (ShortConv + SiLU, L2
   norm per head for q and k, right padding and the decode history);
-* beta: the projection, then ``fused.beta_gate``;
-* decay: the low-rank projection, then ``fused.lower_bounded_decay``, which
+* beta and the decay: their projections, then ``fused.layer_gates``, which
   feeds the operator (the chunk kernel can also form g from the logits
   itself, ``fused.chunkwise_kda_with_decay``, bit-identical but measured
-  slower, so the layer keeps the two launches);
+  slower, so the layer runs two launches);
 * output: ``fused.rmsnorm_gate`` (RMSNorm times the sigmoid gate of the gate
   projection), the output projection, and the mask.
 
@@ -36,10 +35,10 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib, _prep, fused
-from .chunkwise import chunkwise_kda
-from .recurrent import recurrent_kda
+from .chunkwise import checked_chunkwise
+from .recurrent import checked_recurrent
 from .state import KDAState, ShortConvState
-from .utils import validate_attention_mask
+from .utils import checked_lengths, validate_core_inputs
 
 
 @dataclass
@@ -250,7 +249,7 @@ def kda_attention_forward(
         raise ValueError(f"unsupported KDA mode {mode!r}")
     if mode == "decode" and tokens != 1:
         raise ValueError("decode mode requires exactly one token")
-    validate_attention_mask(attention_mask, batch, tokens)
+    valid = checked_lengths(attention_mask, batch, tokens, hidden_states.device)
     _validate_state(w, hidden_states, state)
     x = hidden_states
     if mode == "decode" and attention_mask is None:
@@ -263,13 +262,14 @@ def kda_attention_forward(
     # projections (src/kda/projections.py:164-218)
     qs, ks, vs = (None, None, None) if state is None else (state.q_conv_state, state.k_conv_state,
                                                              state.v_conv_state)
-    q, q_next = fused.conv_silu(F.linear(x, w.q_proj, w.q_proj_bias), w.q_conv, w.q_conv_bias, qs, attention_mask,
-                                num_heads=H, normalize=True, eps=w.eps, output_final_state=return_state)
-    k, k_next = fused.conv_silu(F.linear(x, w.k_proj, w.k_proj_bias), w.k_conv, w.k_conv_bias, ks, attention_mask,
-                                num_heads=H, normalize=True, eps=w.eps, output_final_state=return_state)
-    v, v_next = fused.conv_silu(F.linear(x, w.v_proj, w.v_proj_bias), w.v_conv, w.v_conv_bias, vs, attention_mask,
-                                num_heads=H, output_final_state=return_state)
-    beta = fused.beta_gate(F.linear(x, w.beta_proj, w.beta_bias))
+    conv = fused.conv_silu_with_lengths
+    q, q_next = conv(F.linear(x, w.q_proj, w.q_proj_bias), w.q_conv, w.q_conv_bias, qs, valid, num_heads=H,
+                     normalize=True, eps=w.eps, output_final_state=return_state)
+    k, k_next = conv(F.linear(x, w.k_proj, w.k_proj_bias), w.k_conv, w.k_conv_bias, ks, valid, num_heads=H,
+                     normalize=True, eps=w.eps, output_final_state=return_state)
+    v, v_next = conv(F.linear(x, w.v_proj, w.v_proj_bias), w.v_conv, w.v_conv_bias, vs, valid, num_heads=H,
+                     normalize=False, eps=1e-6, output_final_state=return_state)
+    beta_logits = F.linear(x, w.beta_proj, w.beta_bias)
     decay_logits = F.linear(F.linear(x, w.alpha_down), w.alpha_up).reshape(batch, tokens, H, K)
 
     # the operator (src/kda/kda.py:131-151)
@@ -278,14 +278,15 @@ def kda_attention_forward(
     # the decay kernel, then the operator: measured faster than forming g
     # inside the chunk kernel (fused.chunkwise_kda_with_decay, bit-identical),
     # whose extra VALU work lands on the chunk kernel's latency-bound loaders
-    g, _ = fused.lower_bounded_decay(decay_logits, w.a_log, w.g_min, bias=w.b_alpha)
+    g, beta = fused.layer_gates(decay_logits, w.a_log, w.g_min, w.b_alpha, beta_logits)
+    validate_core_inputs(q, k, v, g, beta, initial, None)
     if mode == "chunkwise":
-        core = chunkwise_kda(q, k, v, g, beta, initial, keep_state, attention_mask,
-                             accumulate_state_in_fp32=w.accumulate_state_in_fp32)
+        core = checked_chunkwise(q, k, v, g, beta, initial, keep_state, attention_mask, valid,
+                                 w.accumulate_state_in_fp32)
     else:
-        core = recurrent_kda(q, k, v, g, beta, initial, keep_state, attention_mask,
-                             accumulate_state_in_fp32=w.accumulate_state_in_fp32,
-                             update_state_in_place=update_state_in_place and mode == "decode" and initial is not None)
+        core = checked_recurrent(q, k, v, g, beta, initial, keep_state, attention_mask, valid,
+                                 w.accumulate_state_in_fp32, update_state_in_place=update_state_in_place
+                                 and mode == "decode" and initial is not None)
 
     # RMSNorm x output gate, output projection, mask (src/kda/kda.py:153-161)
     gated = fused.rmsnorm_gate(core.hidden_states, w.norm_weight, w.eps,
@@ -297,11 +298,12 @@ def kda_attention_forward(
     next_state = None
     if return_state:
         # src/kda/kda.py:163-183
-        if attention_mask is None:
-            lengths = torch.full((batch,), tokens, dtype=torch.long, device=x.device)
+        if valid is not None:
+            offset = valid.to(torch.long) if state is None else state.sequence_offset.to(x.device) + valid
+        elif state is None:
+            offset = torch.full((batch,), tokens, dtype=torch.long, device=x.device)
         else:
-            lengths = attention_mask.sum(dim=1).to(torch.long)
-        offset = lengths if state is None else state.sequence_offset.to(x.device) + lengths
+            offset = state.sequence_offset.to(x.device) + tokens
         next_state = KDAState(recurrent_state=core.final_state, q_conv_state=q_next, k_conv_state=k_next,
                               v_conv_state=v_next, sequence_offset=offset)
     return KDALayerOutput(hidden_states=out, state=next_state)

@@ -20,7 +20,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib, _prep
-from .utils import accumulation_dtype, validate_core_inputs, validate_cu_seqlens
+from .utils import accumulation_dtype, checked_lengths, validate_core_inputs, validate_cu_seqlens
 
 
 @dataclass
@@ -54,9 +54,17 @@ def recurrent_kda(
         offsets = validate_cu_seqlens(cu_seqlens, q.shape[0] if q.ndim == 4 else -1,
                                       q.shape[1] if q.ndim == 4 else -1, attention_mask)
     num_states = None if offsets is None else len(offsets) - 1
-    batch, tokens, heads, key_dim, value_dim = validate_core_inputs(
-        q, k, v, g, beta, initial_state, attention_mask, num_states=num_states
-    )
+    batch, tokens, *_ = validate_core_inputs(q, k, v, g, beta, initial_state, None, num_states=num_states)
+    valid = checked_lengths(attention_mask, batch, tokens, q.device)
+    return checked_recurrent(q, k, v, g, beta, initial_state, output_final_state, attention_mask, valid,
+                             accumulate_state_in_fp32, return_states_per_token, offsets, update_state_in_place)
+
+
+def checked_recurrent(q, k, v, g, beta, initial_state, output_final_state, attention_mask, valid,
+                      accumulate_state_in_fp32, return_states_per_token=False, offsets=None,
+                      update_state_in_place=False) -> KDAOperatorOutput:
+    """``recurrent_kda`` on checked inputs; ``valid``: the mask's int32 lengths."""
+    batch, tokens, heads, key_dim, value_dim = (*q.shape, v.shape[-1])
     if return_states_per_token and offsets is not None:
         raise ValueError("return_states_per_token is not supported with cu_seqlens")
     _lib.require_gpu(q)
@@ -115,7 +123,6 @@ def recurrent_kda(
         )
     else:
         cu = None if offsets is None else _prep.cu_tensor(offsets, device)
-        valid = _prep.valid_lengths(attention_mask, device)
         status = lib.kda_recurrent_fwd(
             qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), gc.data_ptr(), bc.data_ptr(), code,
             _lib.ptr(s_in), _lib.ptr(s_out), scode, out.data_ptr(), _lib.ptr(hist),

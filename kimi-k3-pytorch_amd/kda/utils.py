@@ -12,6 +12,8 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
+
 
 def validate_attention_mask(
     attention_mask: torch.Tensor | None,
@@ -28,11 +30,44 @@ def validate_attention_mask(
         )
     if attention_mask.dtype != torch.bool:
         raise TypeError("attention_mask must be boolean (True means valid)")
+    if attention_mask.is_cuda and attention_mask.numel() > 0:
+        low = int(_device_lengths(attention_mask).cpu().min())
+        if low < 0:
+            raise ValueError("attention_mask must be monotonic right-padding")
+        if require_nonempty and low == 0:
+            raise ValueError("all-padding sequences are not supported")
+        return attention_mask
     if tokens > 1 and bool(((~attention_mask[:, :-1]) & attention_mask[:, 1:]).any()):
         raise ValueError("attention_mask must be monotonic right-padding")
     if require_nonempty and bool((attention_mask.sum(dim=1) == 0).any()):
         raise ValueError("all-padding sequences are not supported")
     return attention_mask
+
+
+def _device_lengths(attention_mask: torch.Tensor) -> torch.Tensor:
+    """Valid length per row of a mask on the GPU (int32; -1 for a row whose
+    valid tokens are no prefix): one launch."""
+    mask = attention_mask.contiguous()
+    batch, tokens = mask.shape
+    lengths = torch.empty(batch, dtype=torch.int32, device=mask.device)
+    _lib.check(_lib.load().kda_mask_lengths(mask.data_ptr(), batch, tokens, lengths.data_ptr(),
+                                            _lib.stream_of(mask.device)))
+    return lengths
+
+
+def checked_lengths(attention_mask: torch.Tensor | None, batch: int, tokens: int,
+                    device: torch.device) -> torch.Tensor | None:
+    """``validate_attention_mask`` and the mask's int32 valid lengths on
+    ``device`` in one launch and one host read for a mask on the GPU."""
+    if attention_mask is None:
+        return None
+    if (attention_mask.is_cuda and attention_mask.shape == (batch, tokens) and attention_mask.dtype == torch.bool
+            and attention_mask.numel() > 0):
+        lengths = _device_lengths(attention_mask)
+        if int(lengths.cpu().min()) > 0:
+            return lengths.to(device)
+    validate_attention_mask(attention_mask, batch, tokens)
+    return attention_mask.to(device=device).sum(dim=1, dtype=torch.int32).contiguous()
 
 
 def validate_core_inputs(q, k, v, g, beta, initial_state, attention_mask, *, num_states: int | None = None):
