@@ -37,6 +37,12 @@ def kernel_inputs(q, k, v, g, beta, work_dtype: torch.dtype):
     the reference's cast does; the kernels then compute in f32 on those
     rounded values, with results in the work dtype.
     """
+    common = q.dtype
+    if (work_dtype == torch.float32 and common in (torch.bfloat16, torch.float16, torch.float32)
+            and k.dtype == common and v.dtype == common and g.dtype == common and beta.dtype == common
+            and q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and g.is_contiguous()
+            and beta.is_contiguous()):
+        return (q, k, v, g, beta), common, torch.float32  # the usual call: as they are
     if work_dtype in (torch.bfloat16, torch.float16):
         q, k, v, g, beta = (t.to(work_dtype) for t in (q, k, v, g, beta))
     tensors = (q, k, v, g, beta)
@@ -65,6 +71,8 @@ def state_arg(initial_state: torch.Tensor | None, arith: torch.dtype,
         return None
     if work_dtype in (torch.bfloat16, torch.float16):
         initial_state = initial_state.to(work_dtype)
+    elif initial_state.dtype == arith and initial_state.is_contiguous():
+        return initial_state
     return initial_state.to(arith).contiguous()
 
 

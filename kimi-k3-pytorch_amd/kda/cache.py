@@ -50,9 +50,26 @@ def gather_rows(tensors: Sequence[torch.Tensor], indices: torch.Tensor | None) -
 
 
 def _gather(tensors: list[torch.Tensor], indices: torch.Tensor | None) -> list[torch.Tensor]:
+    outs, status = _launch_gather(tensors, indices)
+    _check_indices(status, tensors[0].shape[0])
+    return outs
+
+
+# Tensors of the first launch.  The host takes about 2 us per tensor to make the
+# outputs, 90 us for the 40 tensors of eight layers, and the call ends with a wait
+# for the index check: the GPU starts on the first few (a layer's state among
+# them, 40 us of copying at 64 sequences) while the rest are made.
+FIRST_LAUNCH = 5
+
+
+def _launch_gather(tensors: list[torch.Tensor],
+                   indices: torch.Tensor | None) -> tuple[list[torch.Tensor], torch.Tensor | None]:
+    """The gather's outputs and the status its kernels set for an index out of
+    range (None for a copy), to be checked before the outputs are used."""
     device = tensors[0].device
     for t in tensors:
-        _lib.require_gpu(t)
+        if not t.is_cuda:
+            _lib.require_gpu(t)
         if t.device != device:
             raise ValueError("all cache tensors must be on one device")
         if t.ndim == 0:
@@ -69,23 +86,28 @@ def _gather(tensors: list[torch.Tensor], indices: torch.Tensor | None) -> list[t
     n_out = n_src if indices is None else indices.shape[0]
     if n_src == 0 and n_out > 0:
         raise IndexError("index out of range for an empty cache batch")
-    outs = [torch.empty((n_out, *t.shape[1:]), dtype=t.dtype, device=device) for t in tensors]
     if n_out == 0:
-        return outs
+        return [t.new_empty((0, *t.shape[1:])) for t in tensors], None
     lib = _lib.load()
-    n = len(tensors)
-    src = (ctypes.c_void_p * n)(*[t.data_ptr() for t in tensors])
-    dst = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-    row_bytes = (ctypes.c_int64 * n)(*[t[0].numel() * t.element_size() if n_src else 0 for t in tensors])
     status = None if indices is None else torch.zeros(1, dtype=torch.int32, device=device)
-    _lib.check(
-        lib.kda_cache_gather(
-            src, dst, row_bytes, n, _lib.ptr(indices), n_src, n_out, _lib.ptr(status), _prep.stream(device)
-        )
-    )
+    stream, outs = _prep.stream(device), []
+    for group in (tensors[:FIRST_LAUNCH], tensors[FIRST_LAUNCH:]):
+        n = len(group)
+        if n == 0:
+            break
+        new = [t.new_empty((n_out, *t.shape[1:])) for t in group]
+        src = (ctypes.c_void_p * n)(*[t.data_ptr() for t in group])
+        dst = (ctypes.c_void_p * n)(*[o.data_ptr() for o in new])
+        row_bytes = (ctypes.c_int64 * n)(*[t.numel() // n_src * t.element_size() if n_src else 0 for t in group])
+        _lib.check(lib.kda_cache_gather(src, dst, row_bytes, n, _lib.ptr(indices), n_src, n_out, _lib.ptr(status),
+                                        stream))
+        outs += new
+    return outs, status
+
+
+def _check_indices(status: torch.Tensor | None, n_src: int) -> None:
     if status is not None and int(status.item()) != 0:
         raise IndexError(f"index out of range for a cache batch of {n_src}")
-    return outs
 
 
 class _GatherRows(torch.autograd.Function):
@@ -138,8 +160,14 @@ def reorder_states(states: Sequence[KDAState], indices: torch.Tensor) -> list[KD
     flat = [t for s in states for t in _flatten(s)]
     if flat and indices.device != flat[0].device:
         raise ValueError("indices and state must be on the same device")
-    out = gather_rows(flat, indices)
-    return [_rebuild(out[5 * i : 5 * i + 5]) for i in range(len(states))]
+    if not flat or (torch.is_grad_enabled() and any(t.requires_grad for t in flat)):
+        out, status = gather_rows(flat, indices), None
+    else:
+        out, status = _launch_gather([_rows(t) for t in flat], indices)
+    new = [_rebuild(out[5 * i : 5 * i + 5]) for i in range(len(states))]  # while the GPU copies
+    if status is not None:
+        _check_indices(status, flat[0].shape[0])
+    return new
 
 
 def clone_states(states: Sequence[KDAState]) -> list[KDAState]:

@@ -160,7 +160,9 @@ def _forward(q, k, v, g, beta, initial_state, output_final_state, valid, work_dt
 
 
 def needs_grad(*tensors) -> bool:
-    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+    if not torch.is_grad_enabled():
+        return False
+    return any(t is not None and t.requires_grad for t in tensors)
 
 
 def differentiable(q, k, v, g, beta, initial_state, output_final_state, attention_mask, work_dtype, *,
@@ -209,6 +211,8 @@ def _head_group(need, heads) -> int:
     """Heads per kernel call: all of them when the call's workspace,
     need(heads) bytes, fits WORKSPACE_LIMIT, else the most that fit (at least
     one)."""
+    if need(heads) <= WORKSPACE_LIMIT:
+        return heads
     # the size grows with the heads: the largest count that fits, by bisection
     lo, hi = 1, heads
     while lo < hi:

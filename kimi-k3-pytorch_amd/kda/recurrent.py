@@ -69,21 +69,17 @@ def checked_recurrent(q, k, v, g, beta, initial_state, output_final_state, atten
         raise ValueError("return_states_per_token is not supported with cu_seqlens")
     _lib.require_gpu(q)
     work_dtype = accumulation_dtype(v.dtype, accumulate_state_in_fp32)
-    from .chunkwise import differentiable, needs_grad
-
-    if needs_grad(q, k, v, g, beta, initial_state):
+    if _chunkwise.needs_grad(q, k, v, g, beta, initial_state):
         if update_state_in_place:
             raise RuntimeError("the MI355X KDA backward does not support update_state_in_place")
         if return_states_per_token:
-            from .chunkwise import _mask_differentiable
-
-            qm, gm, bm = _mask_differentiable(q, g, beta, attention_mask)
+            qm, gm, bm = _chunkwise._mask_differentiable(q, g, beta, attention_mask)
             hidden, final, hist = _RecurrentStatesFunction.apply(qm, k, v, gm, bm, initial_state, output_final_state,
                                                                  work_dtype)
             return KDAOperatorOutput(hidden_states=hidden, final_state=final if output_final_state else None,
                                      states_per_token=tuple(hist.unbind(0)))
-        return differentiable(q, k, v, g, beta, initial_state, output_final_state, attention_mask, work_dtype,
-                              recurrent=True, offsets=offsets)
+        return _chunkwise.differentiable(q, k, v, g, beta, initial_state, output_final_state, attention_mask,
+                                         work_dtype, recurrent=True, offsets=offsets)
     lib = _lib.load()
 
     (qc, kc, vc, gc, bc), kernel_dtype, arith = _prep.kernel_inputs(q, k, v, g, beta, work_dtype)
@@ -183,3 +179,7 @@ class _RecurrentStatesFunction(torch.autograd.Function):
         grads = [dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg.to(g.dtype), dbeta.to(beta.dtype),
                  None if ds0 is None else ds0.to(initial_state.dtype)]
         return (*[gr if need else None for gr, need in zip(grads, ctx.needs_input_grad[:6])], None, None)
+
+
+# at the end: chunkwise.py imports KDAOperatorOutput from this module
+from . import chunkwise as _chunkwise  # noqa: E402

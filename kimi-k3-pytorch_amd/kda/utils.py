@@ -87,10 +87,11 @@ def validate_core_inputs(q, k, v, g, beta, initial_state, attention_mask, *, num
     value_dim = v.shape[-1]
     if beta.shape != (batch, tokens, heads):
         raise ValueError(f"beta must have shape {(batch, tokens, heads)}, got {tuple(beta.shape)}")
-    tensors = (q, k, v, g, beta)
-    if any(t.device != q.device for t in tensors):
+    device = q.device
+    if k.device != device or v.device != device or g.device != device or beta.device != device:
         raise ValueError("all KDA inputs must be on the same device")
-    if any(not t.dtype.is_floating_point for t in tensors):
+    if not (q.dtype.is_floating_point and k.dtype.is_floating_point and v.dtype.is_floating_point
+            and g.dtype.is_floating_point and beta.dtype.is_floating_point):
         raise TypeError("all KDA inputs must use floating-point dtypes")
     if initial_state is not None:
         lead = batch if num_states is None else num_states
@@ -99,7 +100,7 @@ def validate_core_inputs(q, k, v, g, beta, initial_state, attention_mask, *, num
             raise ValueError(
                 f"initial_state must have shape {expected}, got {tuple(initial_state.shape)}"
             )
-        if initial_state.device != q.device:
+        if initial_state.device != device:
             raise ValueError("initial_state and inputs must be on the same device")
     validate_attention_mask(attention_mask, batch, tokens)
     return batch, tokens, heads, key_dim, value_dim
