@@ -1962,13 +1962,25 @@ static int64_t segment_override() { return g_segment_override.load(std::memory_o
 constexpr double kUnsegChunk = 7.3, kUnsegStart = 6.5, kCutGain = 0.9;
 constexpr double kSegChunk = 11.0, kSegStart = 6.0, kSegLaunches = 7.5, kCombineStep = 0.45, kSegBytes = 0.05;
 
-// `longest` (packed documents only, 0 when unknown): the longest document in
-// tokens.  Documents of uneven length that alone fill the GPU would leave it
-// idle while the longest runs on (one workgroup per document and head); cut
-// into segments, the long chains spread over the CUs the short documents free.
-// Past kModelledSteps chunk steps per CU the model's best is the balanced
-// pass, L = the chunk steps per CU, so no other length is priced there.
+// Packed documents of uneven length: the host knows their number, their
+// tokens and the longest one (`longest`, 0 when unknown), so the documents are
+// taken as the longest, equal others and a quarter as many single chunks (the
+// partial last segments that the equal lengths hide).  What decides there is
+// that the segments fill whole rounds of workgroups: the priced lengths are
+// the shortest that fit one to four rounds, since one workgroup past a round
+// costs a round (documents of 41, 234 and 109 chunks, B x H x 3 = 24 chains,
+// K = V = 64: L = 12 225 us, L = 13 133 us; 10 documents of 9 to 42 chunks at
+// H = 4: L = 4 102 us, L = 5 69 us).  Constants fitted to 126 random document
+// sets (1 to 16 chunk steps per CU, 2 to 12 documents, L forced from 0 to 3
+// times the balanced pass): the picked length takes 1.02 times the best one's
+// time in the mean (a model of fractional rounds 1.13, cutting only past two
+// chunk-workgroups per CU to the balanced pass 1.35).
+// Past kModelledSteps chunk steps per CU the rounds are many and overlap: the
+// balanced pass, L = the chunk steps per CU, is the only length priced.
 constexpr int64_t kModelledSteps = 16;
+constexpr double kDocUnsegStart = 10.0, kDocUnsegChunk = 6.0, kDocLaunches = 10.0, kDocStart = 8.7;
+constexpr double kDocChunk = 7.9, kDocCombineStep = 0.55, kDocSegBytes = 0.045;
+constexpr int64_t kDocRounds = 4;
 static Plan make_plan(int64_t N, int64_t total_tokens, int64_t H, int64_t V, int64_t longest) {
   Plan p;
   p.ncg = (V + kColGroup - 1) / kColGroup;
@@ -1988,7 +2000,7 @@ static Plan make_plan(int64_t N, int64_t total_tokens, int64_t H, int64_t V, int
   p.L = kOneSegment;
   p.segmented = false;
   p.segs_bound = N;
-  if (forced == 0 || N <= 0) return p;
+  if (forced == 0 || N <= 0 || H <= 0 || V <= 0) return p;
   const int64_t span = longest > 0 ? longest : (total_tokens + N - 1) / N;  // the longest sequence (known or even)
   const int64_t n = (span + kChunk - 1) / kChunk;                           // its chunks
   const bool even = N * span <= total_tokens;
@@ -1998,6 +2010,32 @@ static Plan make_plan(int64_t N, int64_t total_tokens, int64_t H, int64_t V, int
   // one chain per (sequence, head, column group) on three quarters of the CUs
   // or more: cutting equal chains only adds a second round and the records
   if (even && 4 * N * H * p.ncg >= 3 * cus) return p;
+  if (!even && longest > 0 && N > 1 && steps <= kModelledSteps) {
+    const int64_t m = ((total_tokens - longest + N - 2) / (N - 1) + kChunk - 1) / kChunk;
+    const int64_t ones = N / 4, docs = N + ones;
+    const int64_t all = n + (N - 1) * m + ones;
+    auto segs_of = [&](int64_t L) { return (n + L - 1) / L + (N - 1) * ((m + L - 1) / L) + ones; };
+    const int64_t rounds = (docs * H * p.ncg + cus - 1) / cus;
+    double chain = all * wgs / cus;  // the longest serial chain of the uncut documents
+    if (rounds > 1 && chain < static_cast<double>(rounds) * all / docs) chain = static_cast<double>(rounds) * all / docs;
+    if (chain < n) chain = n;
+    double best = kCutGain * (kDocUnsegStart + kDocUnsegChunk * chain);
+    for (int64_t r = 1; r <= kDocRounds; ++r) {
+      const int64_t room = r * cus / (H * p.ncg);  // segments that fit r rounds
+      if (room < docs) continue;
+      int64_t L = (all + room - 1) / room;
+      while (segs_of(L) > room) ++L;  // ends: L = max(n, m) leaves `docs` segments
+      if (L >= n) continue;
+      const int64_t nseg = (n + L - 1) / L;
+      const double us = kDocLaunches + r * (kDocStart + kDocChunk * L) + kDocCombineStep * (nseg > 2 ? nseg - 2 : 0) +
+                        kDocSegBytes * segs_of(L) * H * (static_cast<double>(V) / kColGroup);
+      if (us < best) {
+        best = us;
+        segments_of(L);
+      }
+    }
+    return p;
+  }
   const double rounds0 = even ? static_cast<double>((N * H * p.ncg + cus - 1) / cus) * n : steps;
   double best = kCutGain * (kUnsegStart + kUnsegChunk * (n > rounds0 ? n : rounds0));
   const int64_t L1 = steps <= 1 ? 1 : static_cast<int64_t>(steps + 0.999);

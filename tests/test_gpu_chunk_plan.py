@@ -40,6 +40,21 @@ def test_plan_cuts_short_and_few_sequences():
             assert tokens // 64 * heads * 2 >= 512 or need <= _lib.NOALLOC_SCRATCH_BYTES
 
 
+def test_plan_of_uneven_documents_fills_whole_rounds():
+    """Known longest document: the segments of two documents, whose lengths the
+    hint gives exactly, fit whole rounds of 256 workgroups; degenerate sizes
+    plan without a cut."""
+    for heads, long, short in ((4, 9000, 3000), (8, 20000, 5000), (16, 6393, 3416), (32, 6000, 1000)):
+        cut = _plan(2, long + short, long, heads, 64, 64)
+        n, m = -(-long // 64), -(-short // 64)
+        workgroups = (-(-n // cut) - (-m // cut)) * heads
+        assert cut >= 1 and 1 <= -(-workgroups // 256) <= 4
+        shorter = (-(-n // (cut - 1)) - (-m // (cut - 1))) * heads
+        assert -(-shorter // 256) > -(-workgroups // 256), (heads, cut)  # the shortest that fits
+    assert _plan(256, 300, 45, 32, 128, 128) == 0  # more documents than rounds have room for
+    assert _plan(2, 1, 1, 4, 128, 128) == 0  # an empty document
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize(
     "B,T,H,K,V,docs",
@@ -50,6 +65,8 @@ def test_plan_cuts_short_and_few_sequences():
         (3, 600, 24, 128, 128, None),  # as many segments as the CUs take in one round
         (1, 450, 3, 96, 256, None),    # two column groups, padded key channels
         (1, 901, 4, 128, 128, [0, 1, 65, 129, 900, 901]),  # packed: single tokens beside a long document
+        (1, 5000, 4, 64, 64, [0, 1130, 1131, 3000, 4999, 5000]),  # single tokens, several chunks a segment
+        (1, 3300, 16, 128, 128, [0, 2111, 2500, 3300]),  # segments of several chunks, 16 heads
     ],
 )
 def test_planned_schedule_matches_oracle(segments, B, T, H, K, V, docs):
