@@ -149,10 +149,9 @@ int kda_set_segment_chunks(int64_t chunks_per_segment);
  * 16..256.  Other bf16/f16/f32 inputs with K <= 128 and an f32 state take
  * the split-bf16 chunk path: per-chunk operands in a chunk-parallel kernel,
  * the state scan with every product on split operands (x = hi + lo, two bf16
- * each, relative error about 2^-17) and the outputs in a second
- * chunk-parallel kernel; its workspace is B x H x ceil(T/64) records of
- * 240.5 KiB (K = V = 128: the operands the forward scan and the output
- * kernel read, and each chunk's start state and pseudo-values).  Packed documents on that path are gathered into a
+ * each, relative error about 2^-17) and the outputs from that scan; its
+ * workspace is B x H x ceil(T/64) records of 240.5 KiB (K = V = 128: the
+ * scan's operands, and room for each chunk's start state and pseudo-values).  Packed documents on that path are gathered into a
  * zero-padded batch of num_seqs x dense_span tokens (dense_span must be the
  * longest document's length; a smaller one returns KDA_ERR_INVALID_ARGUMENT
  * where the host can tell, and drops tokens past it otherwise) and their

@@ -63,10 +63,11 @@ struct Layout {
 };
 
 // `backward` false: the record of the forward through these kernels (the
-// split-bf16 chunk path), which holds only what prep_kernel writes without dO,
-// the forward scan and out_kernel read (Aqk^T, W, K~^T, Qg^T, U, D, S, Vt:
-// 41% of the backward's record); the offsets of the other records are 0 and
-// nothing of the forward touches them.  `split` false (bf16 and f16 inputs,
+// split-bf16 chunk path), which holds what prep_kernel writes without dO and
+// the forward scan reads (W, K~^T, U, D, and Aqk and Qg row-major in the places
+// of their transposes); the offsets of the other records are 0 and nothing of
+// the forward touches them.  S and Vt stay in the scan's registers: their room
+// belongs to the documented workspace size and is not touched.  `split` false (bf16 and f16 inputs,
 // kSplitOps): the scans' operand records hold their hi plane alone and, in
 // the backward, S, dS and Vt are bf16 (the gradient kernel reads them as bf16
 // operands), which takes the backward's record from 433 to 265 KiB at
@@ -133,10 +134,10 @@ struct Args {
   float* ws;
   int64_t B, T, H, K, V, NC;
   Layout L;
-  // the forward through these kernels (prep_kernel, fscan_kernel, out_kernel)
+  // the forward through these kernels (prep_kernel, the scan's output reruns)
   const int32_t* valid;  // [B] right-padding lengths or null (prep_kernel)
   float* sT;             // [B,H,K,V] final state or null (forward scan)
-  IT* out;               // [B,T,H,V] (out_kernel)
+  IT* out;               // [B,T,H,V] (output reruns)
   // segmented state scans: nseg segments of seglen chunks per sequence,
   // their records (P, Q, start state) at seg, [direction][B*H][nseg]
   float* seg;
@@ -674,7 +675,10 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
           qg[4 * u + e] = ex * qq[e];
         }
       }
-      if (bwd_records) put_split8<kSplitOps<IT>>(ws + a.L.Ktr, kC * KP, r * KP + c0 + cl, kt);  // Kt row-major
+      if (bwd_records)
+        put_split8<kSplitOps<IT>>(ws + a.L.Ktr, kC * KP, r * KP + c0 + cl, kt);  // Kt row-major
+      else
+        put_split8<kSplitOps<IT>>(ws + a.L.Qgt, kC * KP, r * KP + c0 + cl, qg);  // Qg row-major
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         *reinterpret_cast<f32x4*>(&KgS[r * kRS + c0 + cl + 4 * u]) =
@@ -693,7 +697,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
         xq[e] = lgS[(r0 + e) * kQS + col];
       }
       put_split8<kSplitOps<IT>>(ws + a.L.Ktt, kC * KP, c0 * kC + 8 * i8, xk);
-      put_split8<kSplitOps<IT>>(ws + a.L.Qgt, kC * KP, c0 * kC + 8 * i8, xq);
+      if (bwd_records) put_split8<kSplitOps<IT>>(ws + a.L.Qgt, kC * KP, c0 * kC + 8 * i8, xq);
     }
     __syncthreads();
   }
@@ -804,11 +808,11 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     const int r = (4 * i4) >> 6, cc = (4 * i4) & 63;
     *reinterpret_cast<f32x4*>(ws + a.L.A + 4 * i4) = *reinterpret_cast<const f32x4*>(&AS[r * kRC + cc]);
   }
-  for (int i8 = tr; i8 < kC * kC / 8; i8 += kPT) {  // Aqk^T split, eight positions at a time
+  for (int i8 = tr; i8 < kC * kC / 8; i8 += kPT) {  // Aqk^T (the forward alone: Aqk) split, eight elements at a time
     const int r = (8 * i8) >> 6, c0 = (8 * i8) & 63;
     float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = AqkS[(c0 + e) * kRC + r];
+    for (int e = 0; e < 8; ++e) x[e] = bwd_records ? AqkS[(c0 + e) * kRC + r] : AqkS[r * kRC + c0 + e];
     put_split8<kSplitOps<IT>>(ws + a.L.Aqkt, kC * kC, 8 * i8, x);
   }
   __syncthreads();
@@ -961,7 +965,15 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
 //                               writing each chunk's X and R (and the final
 //                               state after the last chunk).
 // The state lives in f32 MFMA accumulators, one 16-column tile per wave.
-// Every product uses split-bf16 operands for f32 inputs
+// The forward alone (the split-bf16 chunk path) takes its outputs from the
+// reruns (kRunOut): O = Qg X + Aqk R from the state and pseudo-values in their
+// registers, X and R in three bf16 parts (f32's 24 bits) against the records'
+// hi and lo, so no product has fewer bits than an f32 MFMA's.  Storing X and R
+// for a chunk-parallel output kernel moved 192 KB more per chunk at K = V = 128
+// and took 89 + 100 us where the output rerun takes 107 (B = 1, T = 8192,
+// H = 16, f32; the call 454 -> 362 us, 1.01 to 1.30 times as fast over 65
+// random f32 calls); 241 of 256 VGPRs, so one block per CU.
+// Every other product uses split-bf16 operands for f32 inputs
 // (x = hi + lo; hi*hi + hi*lo + lo*hi) and single bf16 operands otherwise
 // (kSplitOps: the records' lo planes are then neither written nor read).  An accumulator pair (row tiles 2s,
 // 2s+1) is the B operand of reduction step s with the reduction index
@@ -1057,6 +1069,33 @@ __device__ __forceinline__ f32x4 mfma3(const bf16x8& ah, const bf16x8& al, const
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc, 0, 0, 0);
 }
 
+// x = h + m + r, three bf16 of which together hold f32's 24 bits
+__device__ __forceinline__ void split3_pair(const f32x4& a, const f32x4& b, bf16x8& h, bf16x8& m, bf16x8& r) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x = e < 4 ? a[e & 3] : b[e & 3];
+    __bf16 hh, mm;
+    split_bf16(x, hh, mm);
+    h[e] = hh;
+    m[e] = mm;
+    r[e] = static_cast<__bf16>(x - static_cast<float>(hh) - static_cast<float>(mm));
+  }
+}
+
+// A split record (hi, lo; hi alone when SPLIT is false) times an f32 operand in
+// three parts: every term above 2^-24 of the product.
+template <bool SPLIT>
+__device__ __forceinline__ f32x4 mfma5(const bf16x8& ah, const bf16x8& al, const bf16x8& h, const bf16x8& m,
+                                       const bf16x8& r, f32x4 acc) {
+  if constexpr (SPLIT) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, m, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, h, acc, 0, 0, 0);
+  }
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, r, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, m, acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, h, acc, 0, 0, 0);
+}
+
 // dO of a chunk as the split B operand of the two position steps: lane (i, g)
 // element e of step s holds dO[t0 + 32 s + perm_k(g, e)][col]
 template <class IT>
@@ -1092,8 +1131,10 @@ struct DoFrag {
 };
 
 // Block kinds of seg_kernel: the value columns of a segment's map (Q), its
-// transition columns (P), or the rerun of a segment from its start state.
-constexpr int kSumV = 0, kSumT = 1, kRun = 2;
+// transition columns (P), or the rerun of a segment from its start state,
+// which leaves each chunk's X and R (kRun, for grad_kernel) or, the forward
+// alone, writes the chunk's output (kRunOut).
+constexpr int kSumV = 0, kSumT = 1, kRun = 2, kRunOut = 3;
 
 // Segments per (sequence, head) that a launch of kind MODE runs: every
 // segment for the reruns; all but the last for the value maps; for the
@@ -1102,7 +1143,7 @@ constexpr int kSumV = 0, kSumT = 1, kRun = 2;
 // transposes in reverse order, runs too.
 template <class IT>
 __host__ __device__ inline int seg_blocks(const Args<IT>& a, int mode) {
-  if (mode == kRun) return a.nseg;
+  if (mode == kRun || mode == kRunOut) return a.nseg;
   if (mode == kSumT) return a.ndir == 2 ? a.nseg : a.nseg - 1;
   return a.nseg - 1;
 }
@@ -1112,6 +1153,8 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
   using SL = SegLds<KP>;
   constexpr int NKT = KP / 16, NKS = KP / 32;
   constexpr bool BWD = DIR == 1, TRANS = MODE == kSumT;
+  constexpr bool OUT = MODE == kRunOut, RERUN = MODE == kRun || OUT;
+  static_assert(!OUT || !BWD, "the forward direction writes outputs");
   constexpr bool DO_TERMS = BWD && !TRANS;                            // Aqk^T dO and Qg^T dO
   constexpr bool EXACT_DO = sizeof(IT) == 2 && !__is_same(IT, f16);  // bf16 dO: its lo part is zero
   constexpr bool SPLIT = kSplitOps<IT>;
@@ -1140,7 +1183,7 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
     if constexpr (TRANS) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) X[ct][r] = (16 * ct + 4 * g4 + r == col) ? 1.f : 0.f;
-    } else if constexpr (MODE == kRun) {
+    } else if constexpr (RERUN) {
       if (has) {
         const float* x0 = rec + KP * KP + KP * Vp + opaque(4 * g4 * Vp + col);  // start state from the combine
 #pragma unroll
@@ -1152,7 +1195,8 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
   Rec<kC, KP, SPLIT> ra;   // forward W, backward Kt        [64][KP]
   Rec<KP, kC, SPLIT> rb;   // forward Kt^T, backward W^T    [KP][64]
   Rec<KP, kC, SPLIT> rq;   // backward Qg^T
-  Rec<kC, kC, SPLIT> raq;  // backward Aqk^T
+  Rec<kC, kC, SPLIT> raq;  // backward Aqk^T, outputs Aqk
+  Rec<kC, KP, SPLIT> rqo;  // outputs Qg                    [64][KP]
   float dval = 0.f, lval = 1.f;
   float u[4][4];    // forward value columns: U of the next chunk, accumulator layout
   DoFrag<IT> dof;   // backward value columns: dO of the next chunk
@@ -1169,6 +1213,10 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
         rb.fetch(ws + a.L.Ktt, tid);
         if (tid < KP) dval = ws[a.L.D + tid];
         if (a.ndir == 2 && tid < kC) lval = ws[a.L.live + tid];
+        if constexpr (OUT) raq.fetch(ws + a.L.Aqkt, tid);
+      }
+      if constexpr (OUT) {
+        if (part == 2) rqo.fetch(ws + a.L.Qgt, tid);
       }
       if (part == 2 && !TRANS && has) {
         const float* up = ws + a.L.U + opaque(4 * g4 * Vp + col);
@@ -1208,6 +1256,10 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
       rq.store(sm, SL::fq, tid);
       raq.store(sm, SL::faq, tid);
     }
+    if constexpr (OUT) {
+      rqo.store(sm, SL::fq, tid);
+      raq.store(sm, SL::faq, tid);
+    }
     if (tid < KP) reinterpret_cast<float*>(sm + SL::d)[tid] = dval;
     if (!BWD && tid < kC) reinterpret_cast<float*>(sm + SL::live)[tid] = lval;
     float uc[4][4];
@@ -1233,8 +1285,9 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
     // P = B X (forward B = W, backward B = Kt), plus Aqk^T dO (backward value
     // columns); one fragment pair ahead
     f32x4 P[4];
+    f32x4 O[4];  // outputs: Qg X, then + Aqk R
 #pragma unroll
-    for (int I = 0; I < 4; ++I) P[I] = zero4();
+    for (int I = 0; I < 4; ++I) P[I] = O[I] = zero4();
     {
       bf16x8 xh[NKS], xl[NKS];
 #pragma unroll
@@ -1249,6 +1302,19 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
           if constexpr (SPLIT) fl[(k + 1) & 1] = frag_ld(sm, SL::fa, k + 1, 1, lane);
         }
         P[k / NKS] = mfma3<SPLIT>(fh[k & 1], fl[k & 1], xh[k % NKS], xl[k % NKS], P[k / NKS]);
+      }
+      if constexpr (OUT) {
+#pragma unroll
+        for (int st = 0; st < NKS; ++st) {
+          bf16x8 xm, xr;
+          split3_pair(X[2 * st], X[2 * st + 1], xh[st], xm, xr);
+#pragma unroll
+          for (int I = 0; I < 4; ++I) {
+            const bf16x8 qh = frag_ld(sm, SL::fq, I * NKS + st, 0, lane);
+            const bf16x8 ql = SPLIT ? frag_ld(sm, SL::fq, I * NKS + st, 1, lane) : qh;
+            O[I] = mfma5<SPLIT>(qh, ql, xh[st], xm, xr, O[I]);
+          }
+        }
       }
     }
     if constexpr (DO_TERMS) {
@@ -1310,6 +1376,29 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
           for (int r = 0; r < 4; ++r) ro[(16 * I + r) * Vp] = BWD ? -P[I][r] : P[I][r];
       }
     }
+    if constexpr (OUT) {  // the chunk's output: Aqk is lower triangular, so rows below 32 need no second step
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        bf16x8 ph, pm, pr;
+        split3_pair(P[2 * st], P[2 * st + 1], ph, pm, pr);
+#pragma unroll
+        for (int I = 2 * st; I < 4; ++I) {
+          const bf16x8 qh = frag_ld(sm, SL::faq, I * 2 + st, 0, lane);
+          const bf16x8 ql = SPLIT ? frag_ld(sm, SL::faq, I * 2 + st, 1, lane) : qh;
+          O[I] = mfma5<SPLIT>(qh, ql, ph, pm, pr, O[I]);
+        }
+      }
+      if (col < a.V) {
+        const int64_t step = a.H * a.V;
+        IT* o = a.out + tok(b, t0, a.T, a.H, h) * a.V + opaque(4 * g4 * static_cast<int>(step) + col);
+        const int left = static_cast<int>(a.T - t0 < kC ? a.T - t0 : kC) - 4 * g4;
+#pragma unroll
+        for (int I = 0; I < 4; ++I)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * I + r < left) o[(16 * I + r) * step] = from_compute<IT>(O[I][r]);
+      }
+    }
     // X' = D X + A^T R (forward A = Kt, backward A = W), plus Qg^T dO
     // (backward value columns); one fragment pair ahead
     bf16x8 rh[2], rl[2];
@@ -1358,7 +1447,7 @@ __device__ __forceinline__ void seg_body(const Args<IT>& a, int64_t id, unsigned
     }
   }
   if (!has) return;
-  if constexpr (MODE != kRun) {  // the segment's map: P (transition columns) or Q (value columns)
+  if constexpr (!RERUN) {  // the segment's map: P (transition columns) or Q (value columns)
     float* dst = TRANS ? rec + opaque(4 * g4 * KP + col) : rec + KP * KP + opaque(4 * g4 * Vp + col);
     const int ld = TRANS ? KP : Vp;
 #pragma unroll
@@ -1387,7 +1476,8 @@ __global__ __launch_bounds__(kSC) void seg_kernel(const Args<IT> a) {
   __shared__ __attribute__((aligned(16))) unsigned char sm[SegLds<KP>::bytes];
   const int64_t n = a.B * a.H * seg_blocks(a, MODE);
   const int64_t id = blockIdx.x;
-  if constexpr (MODE == kSumT) {  // the forward's transition maps serve both directions
+  if constexpr (MODE == kSumT || MODE == kRunOut) {
+    // the forward's transition maps serve both directions; outputs are the forward's
     seg_body<IT, KP, MODE, 0>(a, id, sm);
   } else {
     if (a.dir0 == 0 && id < n)
@@ -1537,85 +1627,6 @@ __host__ __device__ inline int64_t seg_floats(int64_t K, int64_t V, int64_t bh, 
   const Layout L = make_layout(K, V);
   return static_cast<int64_t>(ndir) * bh * seg_count(bh, NC, ndir) *
          (static_cast<int64_t>(L.Kp) * L.Kp + 2 * static_cast<int64_t>(L.Kp) * L.Vp);
-}
-
-// ---- the forward through the same chunk operands ------------------------------
-// prep_kernel, then the forward scan alone (which leaves each chunk's start
-// state S and pseudo-values Vt in the workspace and writes the final state),
-// then out_kernel: O = Qg S + Aqk Vt per chunk, all chunks in parallel.  This
-// is the chunkwise prefill for inputs the bf16 MFMA path does not take (f32
-// inputs, key or value dims off its grid), at the split-bf16 accuracy of the
-// scans.
-constexpr int kOT = 512;  // threads of out_kernel: one 16 x 16 output tile per wave and slab
-template <class IT, int KP>
-__global__ __launch_bounds__(kOT) void out_kernel(const Args<IT> a) {
-  __shared__ __attribute__((aligned(16))) float QgT[KP * kRC];  // Qg^T: channel-major, positions contiguous
-  __shared__ __attribute__((aligned(16))) float AqT[kC * kRC];  // Aqk^T
-  __shared__ __attribute__((aligned(16))) float Ss[KP * kSS];   // S slab [channel][32 columns]
-  __shared__ __attribute__((aligned(16))) float Vs[kC * kSS];   // Vt slab [position][32 columns]
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, lg4 = lane >> 4;
-  const int64_t ch = blockIdx.x;
-  const int64_t c = ch % a.NC, bh = ch / a.NC, b = bh / a.H, h = bh % a.H;
-  const int64_t t0 = c * kC;
-  const float* ws = a.ws + ch * a.L.per;
-  // each slab's S and Vt loads go out one slab ahead (the first before the records)
-  WsTile<KP, 32, kOT> ts;
-  WsTile<kC, 32, kOT> tv;
-  ts.fetch(ws + a.L.S, a.L.Vp, 0, tid);
-  tv.fetch(ws + a.L.Vt, a.L.Vp, 0, tid);
-  {  // the split records back to f32, eight elements at a time: Qgt[col * 64 + r] = Qg[r][col],
-     // Aqkt[j * 64 + i] = Aqk[i][j]
-    const __bf16* qg = reinterpret_cast<const __bf16*>(ws + a.L.Qgt);
-    const __bf16* aq = reinterpret_cast<const __bf16*>(ws + a.L.Aqkt);
-    auto unsplit = [&](const __bf16* rec, int n, float* dst) {
-      constexpr int PER = kC * KP / 8 / kOT;  // the larger record (Qg); Aqk takes the first n / 8 items
-      bf16x8 h[PER], l[PER];
-#pragma unroll
-      for (int it = 0; it < PER; ++it) {
-        const int idx = 8 * (tid + kOT * it);
-        if (idx < n) {
-          h[it] = *reinterpret_cast<const bf16x8*>(rec + idx);
-          if constexpr (kSplitOps<IT>) l[it] = *reinterpret_cast<const bf16x8*>(rec + n + idx);
-        }
-      }
-#pragma unroll
-      for (int it = 0; it < PER; ++it) {
-        const int idx = 8 * (tid + kOT * it);
-        if (idx < n) {
-          f32x4 x0, x1;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            x0[e] = static_cast<float>(h[it][e]) + (kSplitOps<IT> ? static_cast<float>(l[it][e]) : 0.f);
-            x1[e] = static_cast<float>(h[it][4 + e]) + (kSplitOps<IT> ? static_cast<float>(l[it][4 + e]) : 0.f);
-          }
-          float* d = dst + (idx >> 6) * kRC + (idx & 63);
-          *reinterpret_cast<f32x4*>(d) = x0;
-          *reinterpret_cast<f32x4*>(d + 4) = x1;
-        }
-      }
-    };
-    unsplit(qg, kC * KP, QgT);
-    unsplit(aq, kC * kC, AqT);
-  }
-  const int rt = w & 3, ct = w >> 2;
-  for (int s0 = 0; s0 < a.L.Vp; s0 += 32) {
-    __syncthreads();  // the previous slab's reads are done
-    ts.template store<kSS>(Ss, tid);
-    tv.template store<kSS>(Vs, tid);
-    if (s0 + 32 < a.L.Vp) {
-      ts.fetch(ws + a.L.S, a.L.Vp, s0 + 32, tid);
-      tv.fetch(ws + a.L.Vt, a.L.Vp, s0 + 32, tid);
-    }
-    __syncthreads();
-    f32x4 acc = mma_long(zero4(), Mat{QgT, 1, kRC}, 16 * rt, Mat{Ss, kSS, 1}, 16 * ct, KP);
-    acc = mma_long(acc, Mat{AqT, 1, kRC}, 16 * rt, Mat{Vs, kSS, 1}, 16 * ct, kC);
-    const int col = s0 + 16 * ct + li;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t t = t0 + 16 * rt + 4 * lg4 + r;
-      if (t < a.T && col < a.V) a.out[tok(b, t, a.T, a.H, h) * a.V + col] = from_compute<IT>(acc[r]);
-    }
-  }
 }
 
 // ---- grad_kernel: every gradient of a chunk from its scan records --------------
@@ -2233,8 +2244,9 @@ static void set_segments(bwd::Args<IT>& a, int ndir) {
   a.seg = a.ws + a.B * a.H * a.NC * a.L.per;
 }
 
-// Both phases and the combine of the segmented scans.
-template <class IT, int KP>
+// Both phases and the combine of the segmented scans; the reruns leave the
+// chunks' records (RUN = kRun) or, the forward alone, outputs (kRunOut).
+template <class IT, int KP, int RUN>
 static void launch_scans(const bwd::Args<IT>& a, hipStream_t s) {
   const int64_t bh = a.B * a.H * a.ndir;
   if (a.nseg > 1 && a.ndir == 2) {  // value maps of both directions and the transition maps together
@@ -2251,7 +2263,7 @@ static void launch_scans(const bwd::Args<IT>& a, hipStream_t s) {
   }
   hipLaunchKernelGGL((bwd::seg_combine_kernel<IT, KP>), dim3(static_cast<unsigned>(a.ndir * bwd::combine_blocks(a))),
                      dim3(bwd::kCT), 0, s, a);
-  hipLaunchKernelGGL((bwd::seg_kernel<IT, KP, bwd::kRun>), dim3(static_cast<unsigned>(bh * a.nseg)), dim3(bwd::kSC),
+  hipLaunchKernelGGL((bwd::seg_kernel<IT, KP, RUN>), dim3(static_cast<unsigned>(bh * a.nseg)), dim3(bwd::kSC),
                      0, s, a);
 }
 
@@ -2260,11 +2272,15 @@ bool chunk_split_path(int in_dtype, int state_dtype, int64_t K, int64_t V) {
          state_dtype == KDA_DTYPE_F32 && K >= 1 && K <= 128 && V >= 1 && V <= 128;
 }
 
+// The forward through the same chunk operands: prep_kernel, then the forward
+// scan alone, whose reruns write the outputs O = Qg S + Aqk Vt from the state
+// and pseudo-values they hold (and the final state).  This is the chunkwise
+// prefill for inputs the bf16 MFMA path does not take (f32 inputs, key or value
+// dims off its grid), at the split-bf16 accuracy of the scans.
 template <class IT, int KP>
 static void launch_split(const bwd::Args<IT>& a, dim3 chunks, hipStream_t s) {
   hipLaunchKernelGGL((bwd::prep_kernel<IT, KP>), chunks, dim3(bwd::kPT), 0, s, a);
-  launch_scans<IT, KP>(a, s);
-  hipLaunchKernelGGL((bwd::out_kernel<IT, KP>), chunks, dim3(bwd::kOT), 0, s, a);
+  launch_scans<IT, KP, bwd::kRunOut>(a, s);
 }
 
 template <class IT>
@@ -2326,7 +2342,7 @@ int launch_chunk_split(const void* q, const void* k, const void* v, const void* 
 template <class IT, int KP>
 static void launch_all(const bwd::Args<IT>& a, dim3 chunks, hipStream_t s) {
   hipLaunchKernelGGL((bwd::prep_kernel<IT, KP>), chunks, dim3(bwd::kPT), 0, s, a);
-  launch_scans<IT, KP>(a, s);
+  launch_scans<IT, KP, bwd::kRun>(a, s);
   const uintptr_t grads = reinterpret_cast<uintptr_t>(a.dq) | reinterpret_cast<uintptr_t>(a.dk) |
                           reinterpret_cast<uintptr_t>(a.dv) | reinterpret_cast<uintptr_t>(a.dg);
   if (a.K == KP && a.V == a.L.Vp && grads % (4 * sizeof(IT)) == 0)
