@@ -148,12 +148,25 @@ def _validate_state(w: KDALayerWeights, hidden_states: torch.Tensor, state: KDAS
         raise ValueError("state and hidden_states must be on the same device")
 
 
-# Largest batch the native decode step takes.  Measured per call at d_model 2048
-# (16 heads x 128, bf16), native against the composed stages: 1 sequence 36 and
-# 301 us (both bound by the host), 32 45 and 293, 128 124 and 294, 256 224 and
-# 274; its projections read the weights again for every 64 sequences, so past
-# 256 the library's GEMMs are the better ones.
+# The calls the native decode step takes: up to DECODE_STEP_BATCH sequences whose
+# projections take at most DECODE_STEP_PRODUCTS multiply-adds.  Its projections
+# read the weights again for every 64 sequences, while the composed stages are
+# bound by the host at about 262 us a call until their GEMMs take longer than
+# that.  Measured per call (us, heads x 128 = d_model, bf16), native against
+# composed:
+#   d_model 2048: 4 sequences 38 / 261, 32 51 / 262, 128 128 / 262, 256 229 / 264;
+#   d_model 4096: 32 101 / 264, 65 (5.5e9 products) 200 / 262, 128 (1.1e10) 298 / 271,
+#     256 556 / 355;
+#   d_model 7168: 4 135 / 265, 32 (8.2e9) 257 / 265, 64 (1.6e10) 418 / 306.
 DECODE_STEP_BATCH = 256
+DECODE_STEP_PRODUCTS = 8_000_000_000
+
+
+def _few_products(w: KDALayerWeights, batch: int) -> bool:
+    """Whether the token's projections keep to DECODE_STEP_PRODUCTS."""
+    weights = (w.q_proj, w.k_proj, w.v_proj, w.beta_proj, w.alpha_down, w.alpha_up, w.gate_proj, w.output_proj)
+    return batch * sum(t.numel() for t in weights) <= DECODE_STEP_PRODUCTS
+
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
@@ -169,7 +182,7 @@ def _decode_step(w: KDALayerWeights, x: torch.Tensor, state: KDAState | None, in
             or K not in (64, 128) or V not in (64, 128) or not w.accumulate_state_in_fp32
             or torch.is_autocast_enabled("cuda") or not w.eps > 0 or not w.g_min < 0):
         return None
-    if any(t.ndim != 2 for t in (w.q_conv, w.alpha_down, w.output_proj)):
+    if any(t.ndim != 2 for t in (w.q_conv, w.alpha_down, w.output_proj)) or not _few_products(w, batch):
         return None
     d_model, kw, vw, taps = x.shape[2], H * K, H * V, w.q_conv.shape[1]
     rank, out_dim = w.alpha_down.shape[0], w.output_proj.shape[0]
