@@ -100,7 +100,11 @@ int kda_decode_step(const void* q, const void* k, const void* v, const void* g,
  * packed documents whose longest is longest_tokens tokens (the value the call
  * passes in `dense_span`; 0 when unknown); off the MFMA path packed documents
  * take a zero-padded batch of num_seqs x longest_tokens tokens, and an
- * f32-state call never needs more.  0 for a longest_tokens outside
+ * f32-state call never needs more.  This is the size of the fastest schedule;
+ * a call with a smaller workspace on the MFMA path runs the balanced schedule
+ * (segments of as many chunks as there are chunk steps per CU) where that one
+ * fits, with results that differ in rounding, and returns KDA_ERR_WORKSPACE
+ * where it does not.  0 for a longest_tokens outside
  * 0..total_tokens.
  * No reference counterpart (the reference allocates per call).
  */
@@ -198,7 +202,8 @@ int kda_chunk_fwd_decay(const void* q, const void* k, const void* v, const void*
  * No counterpart in the reference.  Same arguments, checks and kernels as
  * `kda_chunk_fwd`, minus the workspace: it lives in a static device array of
  * KDA_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the
- * process ends.  A prefill whose workspace exceeds it returns
+ * process ends.  A prefill whose fastest schedule needs more takes the balanced
+ * one where that fits; otherwise it returns
  * KDA_ERR_WORKSPACE before anything is launched (128 MiB covers one
  * 8192-token bf16 sequence at H=16, which needs 72.5 MB; shapes with
  * batch * heads >= 192 need only the small chunk maps; the split-bf16 path's

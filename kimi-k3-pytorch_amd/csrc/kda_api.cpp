@@ -204,7 +204,7 @@ int kda_chunk_fwd(const void* q, const void* k, const void* v, const void* g, co
   if (st != KDA_OK) return st;
   kda::SeqDesc seq{cu_seqlens, dense_span, valid_lens};
   const size_t need = chunk_call_workspace_bytes(seq, num_seqs, total_tokens, heads, key_dim, value_dim, in_dtype,
-                                                 state_dtype);
+                                                 state_dtype, workspace_bytes);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
     set_detail("chunk_fwd needs %zu workspace bytes, got %zu", need, workspace_bytes);
     return KDA_ERR_WORKSPACE;
@@ -237,7 +237,7 @@ int kda_chunk_fwd_decay(const void* q, const void* k, const void* v, const void*
   const int64_t longest = cu_seqlens != nullptr ? dense_span : 0;
   chunk_plan(num_seqs, total_tokens, longest, heads, key_dim, value_dim, in_dtype, &per_segment, &segments);
   const size_t need = per_segment >= 0 ? chunk_workspace_bytes(num_seqs, total_tokens, longest, heads, key_dim,
-                                                               value_dim, in_dtype)
+                                                               value_dim, in_dtype, workspace_bytes)
                                        : 0;
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
     set_detail("chunk_fwd_decay needs %zu workspace bytes, got %zu", need, workspace_bytes);
@@ -264,7 +264,8 @@ int kda_chunk_fwd_profiled(const void* q, const void* k, const void* v, const vo
   st = check_seq(cu_seqlens, dense_span, num_seqs, total_tokens);
   if (st != KDA_OK) return st;
   const size_t need = chunk_call_workspace_bytes(kda::SeqDesc{cu_seqlens, dense_span, valid_lens}, num_seqs,
-                                                 total_tokens, heads, key_dim, value_dim, in_dtype, state_dtype);
+                                                 total_tokens, heads, key_dim, value_dim, in_dtype, state_dtype,
+                                                 workspace_bytes);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
     set_detail("chunk_fwd needs %zu workspace bytes, got %zu", need, workspace_bytes);
     return KDA_ERR_WORKSPACE;

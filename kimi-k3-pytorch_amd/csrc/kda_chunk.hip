@@ -1981,17 +1981,21 @@ constexpr int64_t kModelledSteps = 16;
 constexpr double kDocUnsegStart = 10.0, kDocUnsegChunk = 6.0, kDocLaunches = 10.0, kDocStart = 8.7;
 constexpr double kDocChunk = 7.9, kDocCombineStep = 0.55, kDocSegBytes = 0.045;
 constexpr int64_t kDocRounds = 4;
+
+// Cuts every sequence into segments of L chunks.
+static void cut_into(Plan& p, int64_t L, int64_t N) {
+  p.L = static_cast<int32_t>(L < kOneSegment ? L : kOneSegment - 1);
+  p.segmented = true;
+  p.segs_bound = p.chunks_bound / p.L + N + 1;
+}
+
 static Plan make_plan(int64_t N, int64_t total_tokens, int64_t H, int64_t V, int64_t longest) {
   Plan p;
   p.ncg = (V + kColGroup - 1) / kColGroup;
   const int64_t cus = device_cus();
   const int64_t chunks_bound = total_tokens / kChunk + N;
   p.chunks_bound = chunks_bound;
-  auto segments_of = [&](int64_t L) {
-    p.L = static_cast<int32_t>(L < kOneSegment ? L : kOneSegment - 1);
-    p.segmented = true;
-    p.segs_bound = chunks_bound / p.L + N + 1;
-  };
+  auto segments_of = [&](int64_t L) { cut_into(p, L, N); };
   const int64_t forced = segment_override();
   if (forced > 0) {
     segments_of(forced);
@@ -2076,6 +2080,35 @@ static size_t segment_bytes(const Plan& p, int64_t H, int64_t V) {
   return 2 * st + pp + ma;
 }
 
+static size_t plan_bytes(const Plan& p, int64_t N, int64_t H, int64_t V) {
+  return map_bytes(N) + segment_bytes(p, H, V);
+}
+
+// The plan within `room` bytes of workspace: make_plan's where its records fit.
+// It cuts for time alone, into up to a few times the segments of one balanced
+// pass (N = 24 sequences of 2036 tokens, H = 4, K = V = 128: L = 4 and 175 MiB
+// against L = 12 and 93 MiB), so a smaller workspace, as the 128 MiB scratch of
+// kda_chunk_fwd_noalloc, takes the balanced pass: L = the chunk steps per CU,
+// for sequences that alone leave a quarter of the CUs idle and for packed
+// documents whose longest is well past that length.  Where neither fits, the
+// first, whose size the caller reports.
+static Plan plan_within(int64_t N, int64_t total_tokens, int64_t H, int64_t V, int64_t longest, size_t room) {
+  const Plan p = make_plan(N, total_tokens, H, V, longest);
+  if (segment_override() >= 0 || plan_bytes(p, N, H, V) <= room) return p;
+  Plan q = p;
+  const int64_t cus = device_cus(), work = (total_tokens / kChunk) * H * p.ncg;  // chunk-workgroups of one pass
+  const int64_t steps = (work + cus - 1) / cus, longest_chunks = (longest + kChunk - 1) / kChunk;
+  const bool uneven = N > 1 && 4 * longest_chunks > 5 * steps;
+  if (work >= 2 * cus && (uneven || 4 * N * H * p.ncg < 3 * cus)) {
+    cut_into(q, steps, N);
+  } else {
+    q.L = kOneSegment;
+    q.segmented = false;
+    q.segs_bound = N;
+  }
+  return plan_bytes(q, N, H, V) <= room ? q : p;
+}
+
 static void mark(kda_host::KernelEvents* ev, int i, hipStream_t stream) {
   if (ev != nullptr) {
     (void)hipEventRecord(ev->ev[i], stream);
@@ -2105,9 +2138,8 @@ struct DecayInput {
 template <class IT, bool DECAY, bool PAD, int KT>
 static int run_chunk_k(const void* q, const void* k, const void* v, const void* g, const void* beta, const void* s_in,
                      void* s_out, void* out, const SeqDesc& seq, int64_t N, int64_t total_tokens, int64_t H,
-                     int64_t K, int64_t V, void* workspace, hipStream_t stream, kda_host::KernelEvents* ev,
-                     const DecayInput* decay) {
-  const Plan p = make_plan(N, total_tokens, H, V, plan_longest(seq));
+                     int64_t K, int64_t V, const Plan& p, void* workspace, hipStream_t stream,
+                     kda_host::KernelEvents* ev, const DecayInput* decay) {
   int32_t* chunk_start = static_cast<int32_t*>(workspace);
   int32_t* seg_start = chunk_start + (N + 1);
   unsigned char* segbuf = static_cast<unsigned char*>(workspace) + map_bytes(N);
@@ -2190,18 +2222,18 @@ static int run_chunk_k(const void* q, const void* k, const void* v, const void* 
 template <class IT, bool DECAY>
 static int run_chunk(const void* q, const void* k, const void* v, const void* g, const void* beta, const void* s_in,
                      void* s_out, void* out, const SeqDesc& seq, int64_t N, int64_t total_tokens, int64_t H,
-                     int64_t K, int64_t V, void* workspace, hipStream_t stream, kda_host::KernelEvents* ev,
-                     const DecayInput* decay) {
+                     int64_t K, int64_t V, const Plan& p, void* workspace, hipStream_t stream,
+                     kda_host::KernelEvents* ev, const DecayInput* decay) {
   // K == 128 runs without padding checks; K <= 64 (the reference's shipped
   // model profiles use 64) carries its channels in four row tiles of the state
   if (K == kKey)
     return run_chunk_k<IT, DECAY, false, 8>(q, k, v, g, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V,
-                                            workspace, stream, ev, decay);
+                                            p, workspace, stream, ev, decay);
   if (K <= kKey / 2)
     return run_chunk_k<IT, DECAY, true, 4>(q, k, v, g, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V,
-                                           workspace, stream, ev, decay);
+                                           p, workspace, stream, ev, decay);
   return run_chunk_k<IT, DECAY, true, 8>(q, k, v, g, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V,
-                                         workspace, stream, ev, decay);
+                                         p, workspace, stream, ev, decay);
 }
 
 }  // namespace kda
@@ -2224,7 +2256,7 @@ void chunk_plan(int64_t num_seqs, int64_t total_tokens, int64_t longest, int64_t
 }
 
 size_t chunk_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t longest, int64_t heads,
-                             int64_t key_dim, int64_t value_dim, int in_dtype) {
+                             int64_t key_dim, int64_t value_dim, int in_dtype, size_t room) {
   if (!kda::mfma_path(in_dtype, in_dtype == KDA_DTYPE_F64 ? KDA_DTYPE_F64 : KDA_DTYPE_F32, key_dim, value_dim)) {
     // the split-bf16 chunk path: packed documents (longest > 0) as a padded
     // batch of the longest document's tokens, dense sequences as they are;
@@ -2235,8 +2267,8 @@ size_t chunk_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t lon
     return chunk_split_general_workspace_bytes(num_seqs, (total_tokens + num_seqs - 1) / num_seqs, heads, key_dim,
                                                value_dim, in_dtype, false);
   }
-  const kda::Plan p = kda::make_plan(num_seqs, total_tokens, heads, value_dim, longest);
-  return kda::map_bytes(num_seqs) + kda::segment_bytes(p, heads, value_dim);
+  const kda::Plan p = kda::plan_within(num_seqs, total_tokens, heads, value_dim, longest, room);
+  return kda::plan_bytes(p, num_seqs, heads, value_dim);
 }
 
 // Whether a call off the MFMA path takes the split-bf16 chunk path: a shape
@@ -2250,9 +2282,9 @@ static bool split_call(const kda::SeqDesc& seq, int64_t N, int64_t total_tokens,
 }
 
 size_t chunk_call_workspace_bytes(const kda::SeqDesc& seq, int64_t N, int64_t total_tokens, int64_t H, int64_t K,
-                                  int64_t V, int in_dtype, int state_dtype) {
+                                  int64_t V, int in_dtype, int state_dtype, size_t room) {
   if (kda::mfma_path(in_dtype, state_dtype, K, V))
-    return chunk_workspace_bytes(N, total_tokens, kda::plan_longest(seq), H, K, V, in_dtype);
+    return chunk_workspace_bytes(N, total_tokens, kda::plan_longest(seq), H, K, V, in_dtype, room);
   if (split_call(seq, N, total_tokens, in_dtype, state_dtype, K, V))
     return chunk_split_general_workspace_bytes(N, seq.dense_span, H, K, V, in_dtype, seq.cu_seqlens != nullptr);
   return 0;
@@ -2281,20 +2313,20 @@ int launch_chunk(const void* q, const void* k, const void* v, const void* g, con
     mark(ev, 1, stream);
     return st;
   }
-  if (workspace_bytes < chunk_workspace_bytes(N, total_tokens, plan_longest(seq), H, K, V, in_dtype)) {
+  const Plan p = plan_within(N, total_tokens, H, V, plan_longest(seq), workspace_bytes);
+  if (workspace_bytes < plan_bytes(p, N, H, V)) {
     set_detail("chunk_fwd: workspace too small");
     return KDA_ERR_WORKSPACE;
   }
-  const Plan p = make_plan(N, total_tokens, H, V, plan_longest(seq));
   if (H > 65535 || p.segs_bound * H * p.ncg > 0x7fffffffLL || N > 0x7fffffffLL) {
     set_detail("chunk_fwd: grid too large (N=%lld, H=%lld)", (long long)N, (long long)H);
     return KDA_ERR_UNSUPPORTED;
   }
   if (in_dtype == KDA_DTYPE_BF16)
-    return run_chunk<bf16, false>(q, k, v, g, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, workspace, stream,
-                                  ev, nullptr);
-  return run_chunk<f16, false>(q, k, v, g, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, workspace, stream, ev,
-                               nullptr);
+    return run_chunk<bf16, false>(q, k, v, g, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, p, workspace,
+                                  stream, ev, nullptr);
+  return run_chunk<f16, false>(q, k, v, g, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, p, workspace, stream,
+                               ev, nullptr);
 }
 
 int launch_chunk_decay(const void* q, const void* k, const void* v, const void* z, const void* zbias,
@@ -2307,20 +2339,20 @@ int launch_chunk_decay(const void* q, const void* k, const void* v, const void* 
                "V a multiple of 16 in 16..256); form g with kda_gates_fwd and call kda_chunk_fwd");
     return KDA_ERR_UNSUPPORTED;
   }
-  if (workspace_bytes < chunk_workspace_bytes(N, total_tokens, plan_longest(seq), H, K, V, in_dtype)) {
+  const Plan p = plan_within(N, total_tokens, H, V, plan_longest(seq), workspace_bytes);
+  if (workspace_bytes < plan_bytes(p, N, H, V)) {
     set_detail("chunk_fwd_decay: workspace too small");
     return KDA_ERR_WORKSPACE;
   }
-  const Plan p = make_plan(N, total_tokens, H, V, plan_longest(seq));
   if (H > 65535 || p.segs_bound * H * p.ncg > 0x7fffffffLL || N > 0x7fffffffLL) {
     set_detail("chunk_fwd_decay: grid too large (N=%lld, H=%lld)", (long long)N, (long long)H);
     return KDA_ERR_UNSUPPORTED;
   }
   const DecayInput d{zbias, a_log, g_min};
   if (in_dtype == KDA_DTYPE_BF16)
-    return run_chunk<bf16, true>(q, k, v, z, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, workspace, stream,
-                                 nullptr, &d);
-  return run_chunk<f16, true>(q, k, v, z, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, workspace, stream,
+    return run_chunk<bf16, true>(q, k, v, z, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, p, workspace,
+                                 stream, nullptr, &d);
+  return run_chunk<f16, true>(q, k, v, z, beta, s_in, s_out, out, seq, N, total_tokens, H, K, V, p, workspace, stream,
                               nullptr, &d);
 }
 

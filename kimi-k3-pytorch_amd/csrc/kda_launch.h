@@ -16,9 +16,10 @@ int launch_recurrent(const void* q, const void* k, const void* v, const void* g,
                      bool streaming_state);
 
 // `longest`: the longest packed document in tokens (0 for dense sequences or
-// when unknown), the scheduling hint of make_plan.
+// when unknown), the scheduling hint of make_plan.  `room`: the workspace the
+// call has, which the schedule keeps to where it can (plan_within).
 size_t chunk_workspace_bytes(int64_t num_seqs, int64_t total_tokens, int64_t longest, int64_t heads,
-                             int64_t key_dim, int64_t value_dim, int in_dtype);
+                             int64_t key_dim, int64_t value_dim, int in_dtype, size_t room = SIZE_MAX);
 
 // The schedule launch_chunk picks: chunks per segment (0: one segment per
 // sequence; -1: the exact recurrence kernel) and the bound on segments.
@@ -34,11 +35,11 @@ struct KernelEvents {
   unsigned empty;
 };
 
-// The workspace one launch_chunk call needs: the MFMA path's maps and
-// segment records, the split-bf16 chunk path's per-chunk records, or none
-// (recurrence kernel).
+// The workspace one launch_chunk call needs when it has `room` bytes: the MFMA
+// path's maps and segment records, the split-bf16 chunk path's per-chunk
+// records, or none (recurrence kernel).
 size_t chunk_call_workspace_bytes(const kda::SeqDesc& seq, int64_t N, int64_t total_tokens, int64_t H, int64_t K,
-                                  int64_t V, int in_dtype, int state_dtype);
+                                  int64_t V, int in_dtype, int state_dtype, size_t room);
 
 int launch_chunk(const void* q, const void* k, const void* v, const void* g, const void* beta, int in_dtype,
                  const void* s_in, void* s_out, int state_dtype, void* out, const kda::SeqDesc& seq, int64_t N,
