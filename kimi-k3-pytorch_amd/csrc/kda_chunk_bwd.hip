@@ -1654,7 +1654,7 @@ __host__ __device__ inline int64_t seg_floats(int64_t K, int64_t V, int64_t bh, 
 //
 // Bound: the latency of its phases (about 51 us a workgroup, 20 of it in the
 // slabs, 26 in the quarters); the 256 KB a chunk it must move at K = V = 128 for
-// bf16 would take 95 us over B = 1, T = 8192, H = 16.  66 KB of LDS and at most
+// bf16 would take 95 us over B = 1, T = 8192, H = 16.  71 KB of LDS and at most
 // 128 VGPRs let two workgroups share a CU for bf16 and f16 inputs (f32 inputs
 // keep hi and lo planes: one workgroup; so does bf16 at 256 VGPRs, 65 us slower
 // a call).  Measured there, bf16: 212 us against 354 for the two stages it
@@ -1671,7 +1671,7 @@ struct GradLds {
   static constexpr int dO = dS + planes * KP * kSR * 2;       // bf16 planes x [64][kSR]
   static constexpr int Vt = dO + planes * kC * kSR * 2;
   static constexpr int dv = Vt + planes * kC * kSR * 2;
-  static constexpr int dVf = dv + planes * kC * kSR * 2;      // f32 [64][kSS]
+  static constexpr int dVf = dv + 2 * kC * kSR * 2;           // f32 [64][kSS]; dv keeps both planes for every input
   static constexpr int slab_end = dVf + kC * kSS * 4;
   // second stage, over the first
   static constexpr int dA = 0;                                // f32 [64][kRC]
@@ -2015,13 +2015,15 @@ __global__ __launch_bounds__(kGT, kSplitOps<IT> ? 2 : 4) void grad_kernel(const 
       __bf16 x, y;
       split_bf16(dv, x, y);
       dvs[row * kSR + cl] = x;
-      if constexpr (SPLIT) dvs[pC + row * kSR + cl] = y;
+      dvs[pC + row * kSR + cl] = y;
       if constexpr (!__is_same(IT, bf16)) {
         if (row < rows && (WHOLE || s0 + cl < a.V)) dv0[static_cast<unsigned>(row) * stepV + s0 + cl] = from_compute<IT>(dv);
       }
     }
     __syncthreads();
     fv.load(dvs, pC, 16 * rt, li, g4);
+    bf16x8 dvl;
+    if constexpr (!SPLIT) dvl = *reinterpret_cast<const bf16x8*>(dvs + pC + (16 * rt + li) * kSR + 8 * g4);
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {  // -dKg += dv S^T
       fs.load(Ss, pS, 16 * (2 * j + hf), li, g4);
@@ -2033,6 +2035,10 @@ __global__ __launch_bounds__(kGT, kSplitOps<IT> ? 2 : 4) void grad_kernel(const 
         fb.load(Vts, pC, 16 * (2 * m + hf), li, g4);
         fb.keep(liveB[m]);
         aD[m] = mma_frag<SPLIT>(fv, fb, aD[m]);
+        // single-operand records: dv's second part as well, so that Vt's record
+        // is the product's only rounded operand (dk from dA alone 1.75e-3 off 64
+        // bits, 2.45e-3 with both rounded; 3 us of 694 at B = 1, T = 8192, H = 16)
+        if constexpr (!SPLIT) aD[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dvl, fb.hi, aD[m], 0, 0, 0);
       }
     if constexpr (__is_same(IT, bf16)) {  // dv rounded to bf16 is the tile itself
       const int r = tq >> 3, c4 = (tq & 7) * 4, col = s0 + c4;
