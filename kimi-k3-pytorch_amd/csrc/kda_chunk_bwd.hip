@@ -1981,6 +1981,15 @@ __global__ __launch_bounds__(kGT, kSplitOps<IT> ? 2 : 4) void grad_kernel(const 
 #pragma unroll
       for (int m = 0; m < 2; ++m) liveB[m] = liveS[16 * (2 * m + hf) + li] != 0.f;
     }
+    // f32 inputs: Vt at the E tile's places in all its bits, for dbeta (the LDS
+    // planes hold 16 of them; the 16 KB slab is in the cache).  Ahead of the next
+    // slab's loads, which its wait then leaves in flight.
+    float vf[4];
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        vf[r] = ws[a.L.Vt + s0 + static_cast<unsigned>((16 * rt + 4 * g4 + r) * Vp + 16 * hf + li)];
+    }
     if (s0 + kSW < Vp)
       gs.fetch(a, ws, dO0, stepV, rows, s0 + kSW, tq, WHOLE || (v4 && s0 + 2 * kSW <= a.V));
     // E = N^T dVt, tile (rt, hf) of the slab (N is lower triangular)
@@ -2008,9 +2017,8 @@ __global__ __launch_bounds__(kGT, kSplitOps<IT> ? 2 : 4) void grad_kernel(const 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = 16 * rt + 4 * g4 + r, cl = 16 * hf + li;
-      float e = static_cast<float>(Vts[row * kSR + cl]);
-      if constexpr (SPLIT) e += static_cast<float>(Vts[pC + row * kSR + cl]);
-      db[r] += E[r] * e;
+      if constexpr (SPLIT) db[r] += E[r] * vf[r];
+      else db[r] += E[r] * static_cast<float>(Vts[row * kSR + cl]);
       const float dv = bS[row] * E[r];
       __bf16 x, y;
       split_bf16(dv, x, y);

@@ -50,3 +50,23 @@ def test_strict_product_rounds_one_operand(K, V, T):
     1.8e-3 of the values' norm; two rounded operands err by sqrt(2) as much, from
     2.1e-3 on."""
     assert strict_product_error(K, V, T) < 2.0e-3
+
+
+def beta_gradient_error(H):
+    """dbeta = dO v of single tokens with q = k one channel: v and dO are bf16
+    values and beta has 16 significant bits, so that Vt = beta v is exact in f32
+    and no nearer than 2^-18 in two bf16 parts."""
+    gen = torch.Generator().manual_seed(H)
+    B, K = 8, 64
+    k = torch.zeros(B, 1, H, K)
+    k[..., 3] = 1
+    v, d_out = (torch.randn(B, 1, H, 1, generator=gen).bfloat16().float() for _ in range(2))
+    beta = torch.randint(2**15, 2**16, (B, 1, H), generator=gen).float() / 2**16
+    got, ref = _gradients(k.clone(), k, v, torch.zeros_like(k), beta, d_out)
+    return _rel(got[4], ref[4])
+
+
+def test_f32_beta_gradient_reads_every_bit_of_vt():
+    """f32 inputs: one product, one division and no operand's rounding, each
+    within 2^-24 of its value."""
+    assert beta_gradient_error(64) < 2.0**-23
