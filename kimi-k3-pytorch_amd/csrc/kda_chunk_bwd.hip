@@ -580,7 +580,8 @@ struct QuarterTiles {
 // A row whose beta is zero to f32 (its Vt = beta e underflows against e) still
 // has a beta gradient, E . e.  The backward's records hold e = v - Kg S - A Vt
 // itself on such rows (rows of U and W scaled by one instead of beta) and live
-// = 0, which keeps the row out of every product.
+// = 0, which keeps the row out of every product.  The rows past the end of the
+// sequence have no beta gradient: theirs stay as they are.
 __device__ __forceinline__ bool zero_beta(float b) { return !(fabsf(b) >= 0x1p-100f); }
 
 template <class IT, int KP>
@@ -628,7 +629,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     const int64_t t = t0 + tid;
     const float x = t < Tv ? to_float(a.beta[tok(b, t, a.T, a.H, h)]) : 0.f;
     bS[tid] = x;
-    if (bwd_records) ws[a.L.live + tid] = zero_beta(x) ? 0.f : 1.f;
+    if (bwd_records) ws[a.L.live + tid] = t < Tv && zero_beta(x) ? 0.f : 1.f;
   }
   for (int idx = tid; idx < kC * kRC; idx += kPT) AS[idx] = 0.f;
   // wave w: block pair w, and waves 0 and 1 pairs 8 and 9 as well
@@ -702,7 +703,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     __syncthreads();
   }
   const bool exact = __syncthreads_or(risky);
-  const bool some_zero = bwd_records && __syncthreads_or(tid < kC && zero_beta(bS[tid & (kC - 1)]));
+  const bool some_zero = bwd_records && __syncthreads_or(tid < kC && t0 + tid < Tv && zero_beta(bS[tid & (kC - 1)]));
   if (exact) {
     // A and Aqk with exact pair exponents, 2x2 blocks of (i, j <= i): thread
     // tid takes blocks tid and tid + kPT of the 528, over the quarters again
@@ -872,24 +873,33 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     *reinterpret_cast<f32x4*>(&AS[r * kRC + cc]) = n * *reinterpret_cast<const f32x4*>(&bS[cc]);
   }
   __syncthreads();
-  if (some_zero) {  // rows of zero beta: I - A M in place of M (thread: row tid / 8, columns 8 (tid % 8) ..)
-    const int i = tr >> 3, c8 = (tr & 7) * 8;
-    const bool zero = zero_beta(bS[i]);
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = c8 + e == i ? 1.f : 0.f;
-    if (zero) {
-#pragma unroll 1
-      for (int l = 0; l < i; ++l) {
-        const float al = ws[a.L.A + i * kC + l];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] -= al * AS[l * kRC + c8 + e];
-      }
+  if (some_zero) {
+    // rows of zero beta: I - A M in place of M, wave w the 16x16 tiles w and w + 8
+    // of A M (A from its record, over N).  Masked positions are such rows, so a
+    // right-padded batch has whole chunks of them: the backward of 4 x 2048 tokens,
+    // half masked, H = 16, K = V = 128 bf16 565 us with one chain of reads per
+    // row, 554 like this (539 with none).
+    for (int i4 = tr; i4 < kC * kC / 4; i4 += kPT) {
+      const int r = (4 * i4) >> 6, cc = (4 * i4) & 63;
+      *reinterpret_cast<f32x4*>(&NS[r * kRC + cc]) = *reinterpret_cast<const f32x4*>(ws + a.L.A + 4 * i4);
     }
     __syncthreads();
-    if (zero) {
+    f32x4 z[2];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) AS[i * kRC + c8 + e] = x[e];
+    for (int j = 0; j < 2; ++j) {
+      const int tt = w + 8 * j, rt = tt & 3, ct = tt >> 2;
+      z[j] = zero4();
+      if (ct <= rt) z[j] = mma(zero4(), Mat{NS, kRC, 1}, 16 * rt, Mat{AS, kRC, 1}, 16 * ct, 16 * (rt + 1));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int tt = w + 8 * j, rt = tt & 3, ct = tt >> 2;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * rt + 4 * (lane_id() >> 4) + r, col = 16 * ct + (lane_id() & 15);
+        if (zero_beta(bS[row])) AS[row * kRC + col] = (row == col ? 1.f : 0.f) - z[j][r];
+      }
     }
     __syncthreads();
   }

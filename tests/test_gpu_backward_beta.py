@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import kda
+from kda import _lib
 from oracle import kda_oracle as ora
 from tests._inputs import rel_err, workload
 
@@ -47,3 +48,26 @@ def test_beta_gradient_at_zero_beta(dtype, B, T, H, K, V, zeros):
             assert rel_err(a, r) < TOL[dtype], (name, rel_err(a, r))
         else:
             assert float(a.abs().max()) < 1e-30, name
+
+
+@pytest.mark.parametrize("dtype,K,V", [(torch.bfloat16, 128, 128), (torch.float32, 64, 48)])
+@pytest.mark.parametrize("zeros", [0, 1])
+def test_positions_past_the_end_are_no_zero_beta_rows(dtype, K, V, zeros):
+    """Only a chunk with a real row of zero beta forms those rows' records, for
+    which alone its A (floats 4096 .. 8191 of the chunk's workspace record) is
+    written: the positions past the sequence's end have no beta gradient."""
+    T, H, lib, code = 65, 3, _lib.load(), _lib.dtype_code(dtype)
+    q, k, v, g, beta, _ = (None if t is None else t.to(DEV) for t in workload(1, T, H, K, V, seed=8, dtype=dtype))
+    beta[0, T - 1, 1] *= 1 - zeros  # the last chunk's only row, second head
+    need = lib.kda_chunk_bwd_workspace_bytes(1, T, H, K, V, code)
+    ws = torch.full((need // 4,), float("nan"), device=DEV)
+    grads = [torch.empty_like(t) for t in (q, k, v, g, beta)]
+    _lib.check(lib.kda_chunk_bwd(*(t.data_ptr() for t in (q, k, v, g, beta, torch.ones_like(v))), code, None, None,
+                                 *(t.data_ptr() for t in grads), None, 1, T, H, K, V, ws.data_ptr(), need,
+                                 torch.cuda.current_stream().cuda_stream))
+    assert all(torch.isfinite(t).all() for t in grads)
+    Kp, Vp, s = 64 if K <= 64 else 128, -(-V // 32) * 32, 1 if dtype == torch.float32 else 2
+    rec = 2 * 4096 + 4096 // s + 5 * 64 * Kp // s + 2 * 64 * Vp + Kp + 64 + (2 * Kp * Vp + 64 * Vp) // s
+    records = ws[: 2 * H * (-(-rec // 64) * 64)].reshape(H, 2, -1)  # (head, chunk)
+    written = ~records[:, :, 4096:8192].isnan().all(dim=2)
+    assert written.tolist() == [[False, False], [False, bool(zeros)], [False, False]]
