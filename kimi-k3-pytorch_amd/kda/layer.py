@@ -151,21 +151,47 @@ def _validate_state(w: KDALayerWeights, hidden_states: torch.Tensor, state: KDAS
 # The calls the native decode step takes: up to DECODE_STEP_BATCH sequences whose
 # projections take at most DECODE_STEP_PRODUCTS multiply-adds.  Its projections
 # read the weights again for every 64 sequences, while the composed stages are
-# bound by the host at about 262 us a call until their GEMMs take longer than
+# bound by the host at about 240 us a call until their GEMMs take longer than
 # that.  Measured per call (us, heads x 128 = d_model, bf16), native against
 # composed:
-#   d_model 2048: 4 sequences 38 / 261, 32 51 / 262, 128 128 / 262, 256 229 / 264;
-#   d_model 4096: 32 101 / 264, 65 (5.5e9 products) 200 / 262, 128 (1.1e10) 298 / 271,
-#     256 556 / 355;
-#   d_model 7168: 4 135 / 265, 32 (8.2e9) 257 / 265, 64 (1.6e10) 418 / 306.
+#   d_model 2048: 4 sequences 37 / 238, 32 49 / 239, 128 127 / 239, 256 228 / 242;
+#   d_model 4096: 32 98 / 238, 65 (5.5e9 products) 201 / 239, 128 (1.1e10) 297 / 258,
+#     256 557 / 348;
+#   d_model 7168: 4 134 / 239, 32 (8.3e9) 258 / 254, 64 (1.7e10) 417 / 303.
+# A captured call has no host time: its line is where the device times meet, at
+# 128-wide heads (with key or value heads of 64 the composed stages' device time
+# is the longer one up to DECODE_STEP_PRODUCTS: 1.2 to 2.9 times).  There, replays
+# of the two, native over composed:
+#   d_model 1024: 256 sequences 0.91;  1536: 160 0.94, 192 1.03;
+#   2048: 128 0.88, 192 (3.9e5 activations) 1.06, 256 1.16;  2560: 64 0.83, 128 1.01;
+#   3072: 64 0.83, 96 (2.9e5) 1.09;  4096: 48 0.95, 64 (5.4e9 products) 1.01, 96 1.11;
+#   5120: 32 0.94, 64 1.22;  6144: 24 0.95, 48 1.12;  7168: 16 0.98, 24 (6.2e9) 1.07.
 DECODE_STEP_BATCH = 256
 DECODE_STEP_PRODUCTS = 8_000_000_000
+CAPTURED_STEP_PRODUCTS = 5_000_000_000
+CAPTURED_STEP_ACTIVATIONS = 1 << 18
+
+
+def _products(w: KDALayerWeights, batch: int) -> int:
+    """Multiply-adds of the token's projections."""
+    weights = (w.q_proj, w.k_proj, w.v_proj, w.beta_proj, w.alpha_down, w.alpha_up, w.gate_proj, w.output_proj)
+    return batch * sum(t.numel() for t in weights)
 
 
 def _few_products(w: KDALayerWeights, batch: int) -> bool:
     """Whether the token's projections keep to DECODE_STEP_PRODUCTS."""
-    weights = (w.q_proj, w.k_proj, w.v_proj, w.beta_proj, w.alpha_down, w.alpha_up, w.gate_proj, w.output_proj)
-    return batch * sum(t.numel() for t in weights) <= DECODE_STEP_PRODUCTS
+    return _products(w, batch) <= DECODE_STEP_PRODUCTS
+
+
+def _captured_past_the_line(w: KDALayerWeights, batch: int) -> bool:
+    """Whether the call is being captured into a graph and its replays take
+    longer in the native step than in the composed stages."""
+    if w.key_head_dim != 128 or w.value_head_dim != 128:
+        return False
+    if (batch * w.q_proj.shape[1] <= CAPTURED_STEP_ACTIVATIONS
+            and _products(w, batch) <= CAPTURED_STEP_PRODUCTS):
+        return False
+    return torch.cuda.is_current_stream_capturing()
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
@@ -182,7 +208,9 @@ def _decode_step(w: KDALayerWeights, x: torch.Tensor, state: KDAState | None, in
             or K not in (64, 128) or V not in (64, 128) or not w.accumulate_state_in_fp32
             or torch.is_autocast_enabled("cuda") or not w.eps > 0 or not w.g_min < 0):
         return None
-    if any(t.ndim != 2 for t in (w.q_conv, w.alpha_down, w.output_proj)) or not _few_products(w, batch):
+    if any(t.ndim != 2 for t in (w.q_conv, w.q_proj, w.alpha_down, w.output_proj)):
+        return None
+    if not _few_products(w, batch) or _captured_past_the_line(w, batch):
         return None
     d_model, kw, vw, taps = x.shape[2], H * K, H * V, w.q_conv.shape[1]
     rank, out_dim = w.alpha_down.shape[0], w.output_proj.shape[0]

@@ -109,3 +109,36 @@ def test_calls_the_native_step_leaves_to_the_stages():
     gw.q_conv = gw.q_conv.float()
     with pytest.raises(TypeError, match="weight must have dtype"), torch.no_grad():
         kda_attention_forward(gw, xd, state=state, mode="decode")
+
+
+@pytest.mark.parametrize("B,native", [(32, True), (256, False)])
+def test_captured_step_takes_the_faster_route_and_replays(monkeypatch, B, native):
+    # a large batch: the native step outside a capture, the composed stages
+    # (faster without their host time) inside one; each replay after other work
+    w, gw, x, st = _case(B, 16, 128, 128, 4, 128, torch.bfloat16, False, "head", seed=B)
+    xd, state, step, taken = x.to(DEV), _state(st), layer._decode_step, []
+    monkeypatch.setattr(layer, "_decode_step", lambda *a: taken.append(step(*a)) or taken[-1])
+    with torch.no_grad():
+        ref = kda_attention_forward(gw, xd, state=state, mode="decode")
+        assert taken.pop() is not None
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            monkeypatch.setattr(layer, "DECODE_STEP_BATCH", 0 if not native else 256)  # the route to be captured
+            kda_attention_forward(gw, xd, state=state, mode="decode")
+        torch.cuda.current_stream().wait_stream(side)
+        monkeypatch.setattr(layer, "DECODE_STEP_BATCH", 256)
+        taken.clear()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = kda_attention_forward(gw, xd, state=state, mode="decode")
+        assert (taken.pop() is not None) is native
+        for seed in range(3):
+            xd.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(seed)))
+            ref = kda_attention_forward(gw, xd, state=state, mode="decode")  # eager work between the replays
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert rel_err(got.hidden_states, ref.hidden_states) < 1e-2
+            for i, (a, b) in enumerate(zip(_tuple(got.state), _tuple(ref.state))):
+                assert torch.equal(a, b) if i == 4 or native else rel_err(a, b) < 1e-2, i

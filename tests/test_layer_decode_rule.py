@@ -26,3 +26,18 @@ def _weights(d_model, rank=128):
                                                   (7168, 64, False)])
 def test_size_rule_follows_the_measured_sides(d_model, batch, native):
     assert layer._few_products(_weights(d_model), batch) is native
+
+
+@pytest.mark.parametrize("d_model,batch,composed", [(1024, 256, False), (1536, 192, True), (2048, 128, False),
+                                                    (2048, 129, True), (2048, 256, True), (3072, 64, False),
+                                                    (3072, 96, True), (4096, 48, False), (4096, 64, True),
+                                                    (6144, 24, False), (7168, 16, False), (7168, 24, True)])
+def test_captured_calls_follow_the_device_times(monkeypatch, d_model, batch, composed):
+    w = _weights(d_model)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert layer._captured_past_the_line(w, batch) is composed
+    w.key_head_dim = 64  # the composed stages are slower at every such size
+    assert layer._captured_past_the_line(w, batch) is False
+    w.key_head_dim = 128
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    assert layer._captured_past_the_line(w, batch) is False
