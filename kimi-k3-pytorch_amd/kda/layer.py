@@ -208,6 +208,10 @@ def _decode_step(w: KDALayerWeights, x: torch.Tensor, state: KDAState | None, in
             or K not in (64, 128) or V not in (64, 128) or not w.accumulate_state_in_fp32
             or torch.is_autocast_enabled("cuda") or not w.eps > 0 or not w.g_min < 0):
         return None
+    required = (w.q_proj, w.k_proj, w.v_proj, w.beta_proj, w.alpha_down, w.alpha_up, w.gate_proj, w.output_proj,
+                w.q_conv, w.k_conv, w.v_conv, w.b_alpha, w.a_log)
+    if not batch or any(t is None for t in required):
+        return None  # the stages take a layer without a decay bias, and refuse the rest
     if any(t.ndim != 2 for t in (w.q_conv, w.q_proj, w.alpha_down, w.output_proj)):
         return None
     if not _few_products(w, batch) or _captured_past_the_line(w, batch):

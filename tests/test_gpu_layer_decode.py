@@ -142,3 +142,14 @@ def test_captured_step_takes_the_faster_route_and_replays(monkeypatch, B, native
             assert rel_err(got.hidden_states, ref.hidden_states) < 1e-2
             for i, (a, b) in enumerate(zip(_tuple(got.state), _tuple(ref.state))):
                 assert torch.equal(a, b) if i == 4 or native else rel_err(a, b) < 1e-2, i
+
+
+def test_a_layer_without_decay_bias_keeps_the_stages():
+    w, gw, x, st = _case(3, 2, 64, 64, 4, 16, torch.bfloat16, False, "head", seed=4)
+    gw.b_alpha = torch.zeros_like(gw.b_alpha)
+    with torch.no_grad():
+        ref = kda_attention_forward(gw, x.to(DEV), state=_state(st), mode="decode")
+        gw.b_alpha = None
+        got = kda_attention_forward(gw, x.to(DEV), state=_state(st), mode="decode")
+    assert rel_err(got.hidden_states, ref.hidden_states) < 1e-2
+    assert rel_err(got.state.recurrent_state, ref.state.recurrent_state) < 1e-2
