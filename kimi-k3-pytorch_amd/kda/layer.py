@@ -197,16 +197,23 @@ def _captured_past_the_line(w: KDALayerWeights, batch: int) -> bool:
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+def _transformed() -> bool:
+    """Whether a torch.func transform or a forward-mode level is active: its
+    tensors look like plain ones, and torch's own stages (the projections) take
+    them where a native call does not see them."""
+    return torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+
+
 def _decode_step(w: KDALayerWeights, x: torch.Tensor, state: KDAState | None, in_place: bool) -> KDALayerOutput | None:
     """One token per sequence through ``kda_layer_decode``, or None when the call
-    needs the composed stages: tensors that require grad, autocast, tensor
-    subclasses, layouts, dtypes or sizes the kernels do not take, or anything
+    needs the composed stages: tensors that require grad, autocast, torch.func
+    transforms, tensor subclasses, layouts, dtypes or sizes the kernels do not take, or anything
     the stages would refuse (so that they raise their own errors)."""
     batch, H, K, V = x.shape[0], w.num_heads, w.key_head_dim, w.value_head_dim
     dtype, device = x.dtype, x.device
     if (batch > DECODE_STEP_BATCH or dtype not in (torch.bfloat16, torch.float16) or device.type != "cuda"
             or K not in (64, 128) or V not in (64, 128) or not w.accumulate_state_in_fp32
-            or torch.is_autocast_enabled("cuda") or not w.eps > 0 or not w.g_min < 0):
+            or torch.is_autocast_enabled("cuda") or _transformed() or not w.eps > 0 or not w.g_min < 0):
         return None
     required = (w.q_proj, w.k_proj, w.v_proj, w.beta_proj, w.alpha_down, w.alpha_up, w.gate_proj, w.output_proj,
                 w.q_conv, w.k_conv, w.v_conv, w.b_alpha, w.a_log)

@@ -153,3 +153,26 @@ def test_a_layer_without_decay_bias_keeps_the_stages():
         got = kda_attention_forward(gw, x.to(DEV), state=_state(st), mode="decode")
     assert rel_err(got.hidden_states, ref.hidden_states) < 1e-2
     assert rel_err(got.state.recurrent_state, ref.state.recurrent_state) < 1e-2
+
+
+@pytest.mark.parametrize("transform", ["vmap", "dual"])
+def test_transforms_of_the_output_projection_keep_the_stages(transform):
+    # the output projection is torch's linear: it takes batched and dual weights
+    w, gw, x, st = _case(3, 2, 64, 64, 4, 16, torch.bfloat16, False, "head", seed=6)
+    xd, state, weight = x.to(DEV), _state(st), gw.output_proj
+    other = torch.randn(weight.shape, generator=torch.Generator().manual_seed(2)).to(weight)
+
+    def call(m):
+        gw.output_proj = m
+        return kda_attention_forward(gw, xd, state=state, mode="decode").hidden_states
+
+    with torch.no_grad():
+        one, two = call(weight), call(other)
+        if transform == "vmap":
+            both = torch.vmap(call)(torch.stack([weight, other]))
+            assert rel_err(both[0], one) < 1e-2 and rel_err(both[1], two) < 1e-2
+        else:
+            with torch.autograd.forward_ad.dual_level():
+                got = torch.autograd.forward_ad.unpack_dual(
+                    call(torch.autograd.forward_ad.make_dual(weight, other)))
+            assert rel_err(got.primal, one) < 1e-2 and rel_err(got.tangent, two) < 1e-2
