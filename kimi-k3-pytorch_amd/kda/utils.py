@@ -50,8 +50,9 @@ def _device_lengths(attention_mask: torch.Tensor) -> torch.Tensor:
     mask = attention_mask.contiguous()
     batch, tokens = mask.shape
     lengths = torch.empty(batch, dtype=torch.int32, device=mask.device)
-    _lib.check(_lib.load().kda_mask_lengths(mask.data_ptr(), batch, tokens, lengths.data_ptr(),
-                                            _lib.stream_of(mask.device)))
+    with torch.cuda.device(mask.device):  # a mask may lie on another GPU than the inputs
+        _lib.check(_lib.load().kda_mask_lengths(mask.data_ptr(), batch, tokens, lengths.data_ptr(),
+                                                _lib.stream_of(mask.device)))
     return lengths
 
 
