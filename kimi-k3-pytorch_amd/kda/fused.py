@@ -369,6 +369,11 @@ class _LayerGates(torch.autograd.Function):
         ctx.save_for_backward(logits, a_log, bias, beta_logits)
         ctx.g_min = g_min
         ctx.set_materialize_grads(False)
+        # a gate whose inputs need no gradient has none, as from its own function
+        if not any(ctx.needs_input_grad[:3]):
+            ctx.mark_non_differentiable(g)
+        if not ctx.needs_input_grad[3]:
+            ctx.mark_non_differentiable(beta)
         return g, beta
 
     @staticmethod

@@ -218,3 +218,23 @@ def test_parameter_gradients_under_deterministic_mode():
         assert wg.grad is not None
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("side", ["decay", "beta", "both"])
+def test_layer_gates_differentiate_the_sides_that_need_it(dtype, side):
+    # the one-launch gates as the two functions: a gate without an input that
+    # requires grad does not require it, and the other's gradients are the same
+    z, bl = _rand(2, 5, 3, 16, seed=1).to(DEV, dtype), _rand(2, 5, 3, seed=2).to(DEV, dtype)
+    al, bias = _rand(3, seed=3).to(DEV, torch.float32), _rand(3, 16, seed=4).to(DEV, dtype)
+    decay_leaves = [t.requires_grad_(side != "beta") for t in (z, al, bias)]
+    bl.requires_grad_(side != "decay")
+    g, beta = fused.layer_gates(z, al, -5.0, bias, bl)
+    ref = (fused.lower_bounded_decay(z, al, -5.0, bias=bias)[0], fused.beta_gate(bl))
+    assert torch.equal(g, ref[0]) and torch.equal(beta, ref[1])
+    assert g.requires_grad is (side != "beta") and beta.requires_grad is (side != "decay")
+    leaves = (decay_leaves if side != "beta" else []) + ([bl] if side != "decay" else [])
+    grads = [torch.autograd.grad([t for t in pair if t.requires_grad], leaves,
+                                 [torch.ones_like(t) for t in pair if t.requires_grad]) for pair in ((g, beta), ref)]
+    for a, b in zip(*grads):
+        assert rel_err(a, b) < 1e-5  # atomics sum A_log's and the bias's terms in any order
