@@ -49,7 +49,7 @@ namespace bwd {
 constexpr int kC = 64;     // chunk rows
 constexpr int kRS = 132;   // LDS row stride of [64][<=128] channel matrices
 constexpr int kRC = 68;    // LDS row stride of [64][64] chunk matrices
-constexpr int kSW = 32;    // state columns per slab in grad_body
+constexpr int kSW = 32;    // state columns per slab of grad_kernel
 constexpr int kSS = 36;    // LDS row stride of slab matrices
 constexpr int kTS = 20;    // LDS row stride of 16-column scan tiles
 
@@ -385,31 +385,6 @@ struct RowTile {
     for (int it = 0; it < PER; ++it) {
       const int item = tid + NT * it, r = item / G, c4 = (item % G) * 4;
       *reinterpret_cast<f32x4*>(&dst[r * RS + c4]) = r < rows ? widen<IT>(v[it]) : zero4();
-    }
-  }
-};
-
-// NROW x NCOL f32 of a workspace matrix (row stride ld, from column col0) in
-// registers (fetch), then LDS rows of stride RS (store): the loads go out ahead
-// of the point where the tile is needed.
-template <int NROW, int NCOL, int NT>
-struct WsTile {
-  static constexpr int G = NCOL / 4, PER = NROW * G / NT;
-  static_assert(PER * NT == NROW * G, "the tile must split evenly over the threads");
-  f32x4 v[PER];
-  __device__ __forceinline__ void fetch(const float* src, int ld, int col0, int tid) {
-#pragma unroll
-    for (int it = 0; it < PER; ++it) {
-      const int item = tid + NT * it, r = item / G, c4 = (item % G) * 4;
-      v[it] = *reinterpret_cast<const f32x4*>(src + r * ld + col0 + c4);
-    }
-  }
-  template <int RS>
-  __device__ __forceinline__ void store(float* dst, int tid) const {
-#pragma unroll
-    for (int it = 0; it < PER; ++it) {
-      const int item = tid + NT * it, r = item / G, c4 = (item % G) * 4;
-      *reinterpret_cast<f32x4*>(&dst[r * RS + c4]) = v[it];
     }
   }
 };
@@ -1669,7 +1644,8 @@ __host__ __device__ inline int64_t seg_floats(int64_t K, int64_t V, int64_t bh, 
 // keep hi and lo planes: one workgroup; so does bf16 at 256 VGPRs, 65 us slower
 // a call).  Measured there, bf16: 212 us against 354 for the two stages it
 // replaces (dM, dW and their products with N and A, one workgroup per CU, its
-// 144 KB of gradient records through memory); the whole backward 705 -> 549 us.
+// 144 KB of gradient records through memory); the whole backward 705 -> 554 us
+// (557 with dv in two parts in dA).
 constexpr int kGT = 512;                // threads of grad_kernel
 constexpr int kSR = kSW + 8;            // bf16 row stride of the slab tiles
 template <class IT, int KP>

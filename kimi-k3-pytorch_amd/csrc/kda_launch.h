@@ -74,8 +74,8 @@ int launch_chunk_bwd(const void* q, const void* k, const void* v, const void* g,
                      void* dg, void* dbeta, float* ds0, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V,
                      void* workspace, size_t workspace_bytes, hipStream_t stream);
 
-// The chunkwise forward through the backward's chunk operands (prep, forward
-// scan, output kernel; csrc/kda_chunk_bwd.hip): dense sequences with optional
+// The chunkwise forward through the backward's chunk operands (prep, then the forward
+// scan, which writes the outputs; csrc/kda_chunk_bwd.hip): dense sequences with optional
 // right padding, f32 state, K and V up to 128.
 bool chunk_split_path(int in_dtype, int state_dtype, int64_t K, int64_t V);
 

@@ -5,9 +5,9 @@
 //
 // Reference: KimiDeltaAttention.forward in decode (src/kda/kda.py:98-183) over
 // KDAProjections.forward (src/kda/projections.py:144-225).  The composition of
-// the single stages takes about twenty launches: six skinny GEMMs whose time is
-// the reading of their weights (9 us each for 8 MB at 32 sequences, 1 TB/s) and
-// elementwise kernels of a few microseconds over tensors of a few kilobytes.
+// the single stages takes fifteen launches: eight skinny GEMMs, the large ones
+// bound by the reading of their weights (9 us each for 8 MB at 32 sequences,
+// 1 TB/s), and kernels of a few microseconds over tensors of a few kilobytes.
 // Rounding happens where the stages' tensors round: every projection, q, k, v,
 // beta, z, g, the operator's output and its gated norm are values of the
 // activation type; arithmetic between them is f32, the state f32.
@@ -45,8 +45,9 @@ __device__ __forceinline__ dec_f32x4 mfma8(dec_f16x8 a, dec_f16x8 b, dec_f32x4 c
 // loads of four slices in flight; x comes from L2.  The waves' partial tiles meet
 // in LDS.  With one 32-row tile per workgroup the six projections of a d_model
 // 2048 layer (261 workgroups) fill the CUs in one round.  Measured there at 32
-// sequences: 19.4 us for 43 MB of weights (2.2 TB/s; non-temporal loads 21.9, two
-// slices in flight 20.1), against 67 us in six library GEMMs.
+// sequences: 18.8 us for 34 MB of weights (1.8 TB/s; non-temporal loads 21.9, two
+// slices in flight 20.1), against 53 us in six library GEMMs; the output
+// projection 7.8 us for 8.4 MB (1.1 TB/s), against 9.1.
 constexpr int kLinThreads = 512;
 constexpr int kLinWaves = kLinThreads / 64;
 constexpr int kMaxLinear = 6;
@@ -151,8 +152,8 @@ __global__ __launch_bounds__(kLinThreads) void multi_linear_kernel(const MultiLi
 // [K][V] state tile (held in registers as in recurrent_kernel, its loads issued
 // first), and RMSNorm x output gate.  Bound: the state, read and written once
 // (67 MB, 11 us at 32 sequences of 16 heads, K = V = 128), and the latency of the
-// stages before it: 19 us, against 45 us in nine launches (three ShortConvs,
-// alpha_up, two gates, the recurrence, the norm and the offsets).
+// stages before it: 19 us, against 45 us in eight launches (three ShortConvs,
+// alpha_up, the gates, the recurrence, the norm and the offsets).
 template <class IT>
 struct LayerCore {
   const IT *ql, *kl, *vl, *gl, *bl, *dl;  // projections [B, *]: q, k, v, gate logits, beta logits, alpha_down
