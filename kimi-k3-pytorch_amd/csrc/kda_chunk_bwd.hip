@@ -63,7 +63,7 @@ struct Layout {
 };
 
 // `backward` false: the record of the forward through these kernels (the
-// split-bf16 chunk path), which holds what prep_kernel writes without dO and
+// split-bf16 chunk path), which holds what prep_kernel writes for it and
 // the forward scan reads (W, K~^T, U, D, and Aqk and Qg row-major in the places
 // of their transposes); the offsets of the other records are 0 and nothing of
 // the forward touches them.  S and Vt stay in the scan's registers: their room
@@ -559,7 +559,10 @@ struct QuarterTiles {
 // sequence have no beta gradient: theirs stay as they are.
 __device__ __forceinline__ bool zero_beta(float b) { return !(fabsf(b) >= 0x1p-100f); }
 
-template <class IT, int KP>
+// BWD: the records that only the backward reads (N, Kt row-major, W^T, live) and
+// its rows of zero beta; the forward alone goes without (one kernel for both took
+// the f32 prefill at B = 1, T = 8192, H = 16, K = V = 128 from 365 to 369 us).
+template <class IT, int KP, bool BWD>
 __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
   constexpr int NQ = KP / kQC;  // quarters
   constexpr int NW = KP / 32;   // W tiles per wave
@@ -594,9 +597,6 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     const int64_t n = a.valid[b];
     Tv = n < 0 ? 0 : (n < a.T ? n : a.T);
   }
-  // the records only the backward reads (N, Kt row-major, W^T, live) are
-  // skipped when the kernels serve the forward alone (no dO)
-  const bool bwd_records = a.dout != nullptr;
 
   QuarterTiles<IT> in;
   in.fetch(a, b, t0, h, 0, tid);
@@ -604,7 +604,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     const int64_t t = t0 + tid;
     const float x = t < Tv ? to_float(a.beta[tok(b, t, a.T, a.H, h)]) : 0.f;
     bS[tid] = x;
-    if (bwd_records) ws[a.L.live + tid] = t < Tv && zero_beta(x) ? 0.f : 1.f;
+    if (BWD) ws[a.L.live + tid] = t < Tv && zero_beta(x) ? 0.f : 1.f;
   }
   for (int idx = tid; idx < kC * kRC; idx += kPT) AS[idx] = 0.f;
   // wave w: block pair w, and waves 0 and 1 pairs 8 and 9 as well
@@ -649,9 +649,12 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
           kg[4 * u + e] = ex * kk[e];
           kt[4 * u + e] = fast_exp(la[e] - ll[e]) * kk[e];
           qg[4 * u + e] = ex * qq[e];
+          // the stored product is an f32 value (not one merged with its split's
+          // subtraction), the same one that goes to the transposed record
+          asm volatile("" : "+v"(BWD ? kt[4 * u + e] : qg[4 * u + e]));
         }
       }
-      if (bwd_records)
+      if (BWD)
         put_split8<kSplitOps<IT>>(ws + a.L.Ktr, kC * KP, r * KP + c0 + cl, kt);  // Kt row-major
       else
         put_split8<kSplitOps<IT>>(ws + a.L.Qgt, kC * KP, r * KP + c0 + cl, qg);  // Qg row-major
@@ -673,12 +676,12 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
         xq[e] = lgS[(r0 + e) * kQS + col];
       }
       put_split8<kSplitOps<IT>>(ws + a.L.Ktt, kC * KP, c0 * kC + 8 * i8, xk);
-      if (bwd_records) put_split8<kSplitOps<IT>>(ws + a.L.Qgt, kC * KP, c0 * kC + 8 * i8, xq);
+      if (BWD) put_split8<kSplitOps<IT>>(ws + a.L.Qgt, kC * KP, c0 * kC + 8 * i8, xq);
     }
     __syncthreads();
   }
   const bool exact = __syncthreads_or(risky);
-  const bool some_zero = bwd_records && __syncthreads_or(tid < kC && t0 + tid < Tv && zero_beta(bS[tid & (kC - 1)]));
+  const bool some_zero = BWD && __syncthreads_or(tid < kC && t0 + tid < Tv && zero_beta(bS[tid & (kC - 1)]));
   if (exact) {
     // A and Aqk with exact pair exponents, 2x2 blocks of (i, j <= i): thread
     // tid takes blocks tid and tid + kPT of the 528, over the quarters again
@@ -788,7 +791,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
     const int r = (8 * i8) >> 6, c0 = (8 * i8) & 63;
     float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = bwd_records ? AqkS[(c0 + e) * kRC + r] : AqkS[r * kRC + c0 + e];
+    for (int e = 0; e < 8; ++e) x[e] = BWD ? AqkS[(c0 + e) * kRC + r] : AqkS[r * kRC + c0 + e];
     put_split8<kSplitOps<IT>>(ws + a.L.Aqkt, kC * kC, 8 * i8, x);
   }
   __syncthreads();
@@ -844,7 +847,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
   for (int i4 = tr; i4 < kC * kC / 4; i4 += kPT) {  // M = N diag(b) over A, four at a time
     const int r = (4 * i4) >> 6, cc = (4 * i4) & 63;
     const f32x4 n = *reinterpret_cast<const f32x4*>(&NS[r * kRC + cc]);
-    if (bwd_records) *reinterpret_cast<f32x4*>(ws + a.L.N + 4 * i4) = n;
+    if (BWD) *reinterpret_cast<f32x4*>(ws + a.L.N + 4 * i4) = n;
     *reinterpret_cast<f32x4*>(&AS[r * kRC + cc]) = n * *reinterpret_cast<const f32x4*>(&bS[cc]);
   }
   __syncthreads();
@@ -903,7 +906,7 @@ __global__ __launch_bounds__(kPT, 4) void prep_kernel(const Args<IT> a) {
       y[e] = KgS[(r2 + e) * kRS + c2];
     }
     put_split8<kSplitOps<IT>>(ws + a.L.Wr, kC * KP, 8 * i8, x);
-    if (bwd_records) {
+    if (BWD) {
       if (some_zero) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[e] = zero_beta(bS[r2 + e]) ? 0.f : y[e];
@@ -2279,7 +2282,7 @@ bool chunk_split_path(int in_dtype, int state_dtype, int64_t K, int64_t V) {
 // dims off its grid), at the split-bf16 accuracy of the scans.
 template <class IT, int KP>
 static void launch_split(const bwd::Args<IT>& a, dim3 chunks, hipStream_t s) {
-  hipLaunchKernelGGL((bwd::prep_kernel<IT, KP>), chunks, dim3(bwd::kPT), 0, s, a);
+  hipLaunchKernelGGL((bwd::prep_kernel<IT, KP, false>), chunks, dim3(bwd::kPT), 0, s, a);
   launch_scans<IT, KP, bwd::kRunOut>(a, s);
 }
 
@@ -2341,7 +2344,7 @@ int launch_chunk_split(const void* q, const void* k, const void* v, const void* 
 
 template <class IT, int KP>
 static void launch_all(const bwd::Args<IT>& a, dim3 chunks, hipStream_t s) {
-  hipLaunchKernelGGL((bwd::prep_kernel<IT, KP>), chunks, dim3(bwd::kPT), 0, s, a);
+  hipLaunchKernelGGL((bwd::prep_kernel<IT, KP, true>), chunks, dim3(bwd::kPT), 0, s, a);
   launch_scans<IT, KP, bwd::kRun>(a, s);
   const uintptr_t grads = reinterpret_cast<uintptr_t>(a.dq) | reinterpret_cast<uintptr_t>(a.dk) |
                           reinterpret_cast<uintptr_t>(a.dv) | reinterpret_cast<uintptr_t>(a.dg);
