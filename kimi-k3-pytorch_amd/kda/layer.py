@@ -186,12 +186,9 @@ def _few_products(w: KDALayerWeights, batch: int) -> bool:
 def _captured_past_the_line(w: KDALayerWeights, batch: int) -> bool:
     """Whether the call is being captured into a graph and its replays take
     longer in the native step than in the composed stages."""
-    if w.key_head_dim != 128 or w.value_head_dim != 128:
+    if w.key_head_dim != 128 or w.value_head_dim != 128 or not torch.cuda.is_current_stream_capturing():
         return False
-    if (batch * w.q_proj.shape[1] <= CAPTURED_STEP_ACTIVATIONS
-            and _products(w, batch) <= CAPTURED_STEP_PRODUCTS):
-        return False
-    return torch.cuda.is_current_stream_capturing()
+    return batch * w.q_proj.shape[1] > CAPTURED_STEP_ACTIVATIONS or _products(w, batch) > CAPTURED_STEP_PRODUCTS
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
@@ -215,11 +212,13 @@ def _decode_step(w: KDALayerWeights, x: torch.Tensor, state: KDAState | None, in
             or K not in (64, 128) or V not in (64, 128) or not w.accumulate_state_in_fp32
             or torch.is_autocast_enabled("cuda") or _transformed() or not w.eps > 0 or not w.g_min < 0):
         return None
-    required = (w.q_proj, w.k_proj, w.v_proj, w.beta_proj, w.alpha_down, w.alpha_up, w.gate_proj, w.output_proj,
-                w.q_conv, w.k_conv, w.v_conv, w.b_alpha, w.a_log)
-    if not batch or any(t is None for t in required):
-        return None  # the stages take a layer without a decay bias, and refuse the rest
-    if any(t.ndim != 2 for t in (w.q_conv, w.q_proj, w.alpha_down, w.output_proj)):
+    if not batch:
+        return None
+    for t in (w.q_proj, w.k_proj, w.v_proj, w.beta_proj, w.alpha_down, w.alpha_up, w.gate_proj, w.output_proj,
+              w.q_conv, w.k_conv, w.v_conv, w.b_alpha, w.a_log):
+        if t is None:  # the stages take a layer without a decay bias, and refuse the rest
+            return None
+    if w.q_conv.ndim != 2 or w.q_proj.ndim != 2 or w.alpha_down.ndim != 2 or w.output_proj.ndim != 2:
         return None
     if not _few_products(w, batch) or _captured_past_the_line(w, batch):
         return None
